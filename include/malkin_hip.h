@@ -284,8 +284,8 @@ int mk_penalize(mk_ctx* ctx, float* logits, int64_t stride, const int32_t* rows,
                 const int32_t* pen_off, const int32_t* pen_id, const float* pen_amt);
 /* The top-k cut of Sampler::distribution (sampler.cpp:32-36, std::partial_sort by value): per row the k largest
    logits, highest first, into values / ids [n_rows][k]. k = 1..1024 and at most n_vocab. Equal logits are ordered
-   by lower id (the reference leaves their order unspecified). One workgroup per row: radix select of the k-th
-   largest value, then a sort of the k candidates in LDS. */
+   by lower id (the reference leaves their order unspecified). Rows past 8192 logits are selected from in slices whose
+   candidates go through the context's scratch (no allocation). */
 int mk_topk(mk_ctx* ctx, const float* logits, int64_t stride, const int32_t* rows, int n_rows, int n_vocab, int k,
             float* values, int32_t* ids);
 /* Per-row parameters of mk_sample_cut: candidates k (<= 0: the whole vocabulary) and the request's temperature

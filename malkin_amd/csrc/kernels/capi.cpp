@@ -482,7 +482,7 @@ int mk_topk(mk_ctx* c, const float* logits, int64_t stride, const int32_t* rows,
             float* values, int32_t* ids) {
   return guard([&] {
     require(logits && values && ids && n_rows >= 0 && n_vocab > 0 && stride >= n_vocab, "topk: bad arguments");
-    mk::topk(c->stream, logits, stride, rows, n_rows, n_vocab, k, values, ids);
+    mk::topk(c->stream, logits, stride, rows, n_rows, n_vocab, k, values, ids, c->scratch, c->scratch_bytes);
   });
 }
 

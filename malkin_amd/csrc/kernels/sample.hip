@@ -4,23 +4,39 @@
 // The host finishes the distribution over those k candidates (temperature, min-p, top-p, normalisation, draw), so a
 // sampled request downloads k (value, id) pairs per row instead of the 608 KB logits row.
 //
-// Top-k per row, one 1024-thread workgroup: the logits become order-preserving 32-bit keys; an MSB-first radix
-// select (four 8-bit digits, a 256-bin LDS histogram each) finds the k-th largest key T and how many keys exceed it;
-// the keys above T are collected, then the lowest-indexed keys equal to T in index order; a bitonic sort in LDS
-// orders the k candidates by (key desc, id asc).
+// Top-k per row: the logits become order-preserving 32-bit keys, and a workgroup selects the first of the keys that its
+// threads hold in registers (select_k: a search for the k-th largest key, two bits per step, counted by wave ballots).
+// A long row is cut into kSlices slices of every kSlices-th 64-logit chunk, one workgroup each (k_topk_part); each
+// gives its slice_keep(k) first candidates through the context's scratch, and one workgroup per row selects from those
+// and sorts (k_topk_final). Neighbouring ids fall into different slices, so a slice holds about k / kSlices of the
+// row's first k; where all the candidates of a slice were selected, it may hold more, and the row is then walked
+// whole, in rounds of as many logits as the threads hold.
+// What bounds it: two launches and the searches' barriers; the logits are read once (4.9 MB for 8 rows of 151936). See
+// topk() for the times.
+#include <algorithm>
+
 #include "ctx.h"
 #include "ops.h"
 
 namespace mk {
 namespace {
 
-constexpr int kSelThreads = 1024;
-constexpr int kMaxTopK = 1024;  // candidates per row held in LDS
+constexpr int kSelThreads = 1024;            // k_topk_final
+constexpr int kPartThreads = 256;            // k_topk_part
+constexpr int kPartPer = 16;                 // logits per thread and round of k_topk_part
+constexpr int kFinalPer = 8;                 // keys per thread (and round) of k_topk_final
+constexpr int kMaxTopK = 1024;               // candidates per row held in LDS
+constexpr int kSlices = 64, kChunk = 64;     // slice p of a row: its chunks p, p + kSlices, ...
+constexpr int kOneSlice = kFinalPer * kSelThreads;  // logits of a row that one workgroup takes alone
 
-// Larger float -> larger key (finite values and infinities; NaN logits are not expected).
+// Candidates that a slice gives: four times the k / kSlices it holds on average, and 16.
+__host__ __device__ constexpr int slice_keep(int k) { return k < 16 + k / 16 ? k : 16 + k / 16; }
+static_assert(kSlices * slice_keep(kMaxTopK) <= kFinalPer * kSelThreads, "one workgroup holds a row's candidates");
+
+// Larger float -> larger key, never 0 (finite values and infinities; NaN logits are not expected).
 __device__ __forceinline__ uint32_t order_key(float f) {
   const uint32_t u = __float_as_uint(f);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+  return max((u & 0x80000000u) ? ~u : (u | 0x80000000u), 1u);
 }
 
 // One row per block: l[pen_id[i]] -= pen_amt[i] for this row's entries pen_off[r] .. pen_off[r + 1].
@@ -35,95 +51,211 @@ __global__ void k_penalize(float* __restrict__ logits, int64_t stride, const int
   }
 }
 
-__global__ __launch_bounds__(kSelThreads) void k_topk(const float* __restrict__ logits, int64_t stride,
-                                                       const int32_t* __restrict__ rows, int n_vocab, int k,
-                                                       float* __restrict__ out_v, int32_t* __restrict__ out_i) {
-  __shared__ uint32_t hist[256];
-  __shared__ uint32_t prefix_s, remain_s, count_s;
+// The k-th largest of the workgroup's keys (E per thread), i.e. the largest T with at least k keys >= T: two bits per
+// step from the top, the counts of the three candidate values by wave ballots and one LDS add per wave. cnt: kSteps
+// groups of 3 zeroed counters, fresh ones per step, so that one barrier per step suffices. k >= 1; keys >= k.
+constexpr int kSteps = 16;
+template <int E>
+__device__ __forceinline__ uint32_t kth_largest(const uint32_t (&key)[E], uint32_t k, uint32_t* cnt) {
+  uint32_t T = 0;
+  for (int st = 0; st < kSteps; ++st) {
+    const int shift = 30 - 2 * st;
+    uint32_t c[3] = {0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+#pragma unroll
+      for (int v = 0; v < 3; ++v) c[v] += (uint32_t)__popcll(__ballot(key[e] >= (T | ((uint32_t)(v + 1) << shift))));
+    if ((threadIdx.x & 63) < 3) {
+      const uint32_t own = (threadIdx.x & 63) == 0 ? c[0] : (threadIdx.x & 63) == 1 ? c[1] : c[2];
+      if (own) atomicAdd(&cnt[3 * st + (threadIdx.x & 63)], own);
+    }
+    __syncthreads();
+    const uint32_t *g = cnt + 3 * st;
+    const uint32_t v = g[2] >= k ? 3u : g[1] >= k ? 2u : g[0] >= k ? 1u : 0u;
+    T |= v << shift;
+  }
+  return T;
+}
+
+// LDS of one selection.
+struct SelLds {
+  uint32_t cnt[2][3 * kSteps];  // the counters of the two searches
+  uint32_t gt, eq, slot;
+};
+
+// put(slot, key, id) for the k first keys of the workgroup in the order (key desc, id asc), slots in any order. Threads
+// without a key hold (0, INT32_MAX), below every logit's key; where fewer than k hold one, T is 0, every key is put and
+// some slots are k or more (put drops those, and keys of 0 come last in no order: see below).
+template <int E, class Put>
+__device__ __forceinline__ int select_k(const uint32_t (&key)[E], const int32_t (&id)[E], int k, SelLds& L, Put put) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (tid < 2 * 3 * kSteps) (&L.cnt[0][0])[tid] = 0;
+  if (tid == 0) L.gt = L.eq = L.slot = 0;
+  __syncthreads();
+  const uint32_t T = kth_largest(key, (uint32_t)k, L.cnt[0]);
+  uint32_t ngt = 0, neq = 0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    ngt += (uint32_t)__popcll(__ballot(key[e] > T));
+    neq += (uint32_t)__popcll(__ballot(key[e] == T));
+  }
+  if (lane == 0) {
+    if (ngt) atomicAdd(&L.gt, ngt);
+    if (neq) atomicAdd(&L.eq, neq);
+  }
+  __syncthreads();
+  // Of the keys equal to T, the need lowest ids: those with ~id at least the need-th largest ~id among them.
+  const uint32_t need = (uint32_t)k - L.gt;
+  uint32_t U = 0;
+  if (T != 0 && L.eq > need) {
+    uint32_t inv[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) inv[e] = key[e] == T ? ~(uint32_t)id[e] : 0u;
+    U = kth_largest(inv, need, L.cnt[1]);
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const bool take = key[e] > T || (T != 0 && key[e] == T && ~(uint32_t)id[e] >= U);
+    const unsigned long long bal = __ballot(take);
+    if (bal == 0) continue;
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(&L.slot, (uint32_t)__popcll(bal));
+    base = (uint32_t)__shfl((int)base, 0);
+    if (take) put(base + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull)), key[e], id[e]);
+  }
+  return T != 0 ? k : (int)L.gt;
+}
+
+// Slice p of a row: its slice_keep(k) first candidates (all of them, then (0, INT32_MAX), where it holds no more) to
+// cand[row][p][keep]. A slice of more logits than the threads hold is walked in rounds, each over the candidates so far
+// and the next logits.
+__global__ __launch_bounds__(kPartThreads) void k_topk_part(const float* __restrict__ logits, int64_t stride,
+                                                             const int32_t* __restrict__ rows, int n_vocab, int keep,
+                                                             uint2* cand) {
+  constexpr int E = kPartPer, NT = kPartThreads;
+  __shared__ SelLds L;
+  const int tid = threadIdx.x, r = blockIdx.y, p = blockIdx.x;
+  const float* l = logits + (int64_t)(rows ? rows[r] : r) * stride;
+  auto at = [&](int j) { return ((int64_t)(j / kChunk) * kSlices + p) * kChunk + j % kChunk; };  // slice logit j
+  const int n = (int)((n_vocab + (int64_t)kSlices * kChunk - 1) / (kSlices * kChunk)) * kChunk;  // some past n_vocab
+  uint2* out = cand + ((int64_t)r * kSlices + p) * keep;
+  uint32_t key[E];
+  int32_t id[E];
+  for (int pos = 0, held = 0;;) {  // held: entries of out that join this round (0, then keep)
+    const int take = min(n - pos, E * NT - held);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = e * NT + tid, j = i - held;
+      const int64_t v = at(pos + j);
+      const bool in = j >= 0 && j < take && v < n_vocab;
+      const uint2 old = i < held ? out[i] : make_uint2(0u, (uint32_t)INT32_MAX);
+      id[e] = in ? (int32_t)v : (int32_t)old.y;
+      key[e] = in ? order_key(l[v]) : old.x;
+    }
+    __syncthreads();  // out has been read
+    const int got =
+        select_k(key, id, keep, L, [&](uint32_t slot, uint32_t kk, int32_t ii) { out[slot] = make_uint2(kk, (uint32_t)ii); });
+    for (int i = got + tid; i < keep; i += NT) out[i] = make_uint2(0u, (uint32_t)INT32_MAX);
+    pos += take;
+    if (pos >= n) return;
+    held = keep;
+    __syncthreads();  // out has been written, L has been read
+  }
+}
+
+// One row's k first, sorted: from its slices' candidates (cand[row][kSlices][keep]), or from the row itself (cand NULL;
+// also where a slice's candidates were all selected), in rounds of the keys the threads hold and the best so far.
+__global__ __launch_bounds__(kSelThreads) void k_topk_final(const float* __restrict__ logits, int64_t stride,
+                                                             const int32_t* __restrict__ rows, int n_vocab,
+                                                             const uint2* __restrict__ cand, int k,
+                                                             float* __restrict__ out_v, int32_t* __restrict__ out_i) {
+  constexpr int E = kFinalPer, NT = kSelThreads;
+  __shared__ SelLds L;
   __shared__ uint32_t ckey[kMaxTopK];
   __shared__ int32_t cidx[kMaxTopK];
-  __shared__ uint32_t scan[kSelThreads / 64];
-  const int tid = threadIdx.x;
-  const int r = blockIdx.x;
-  const float* l = logits + (int64_t)(rows ? rows[r] : r) * stride;
-
-  // Radix select: after digit d, `prefix` holds the top 8 (d + 1) bits of T and `remain` the rank of T among the
-  // keys that share them (1 = the largest).
-  if (tid == 0) {
-    prefix_s = 0;
-    remain_s = (uint32_t)k;
-  }
-  for (int d = 0; d < 4; ++d) {
-    const int shift = 24 - 8 * d;
-    const uint32_t hmask = d == 0 ? 0u : 0xFFFFFFFFu << (32 - 8 * d);
-    if (tid < 256) hist[tid] = 0;
-    __syncthreads();
-    const uint32_t prefix = prefix_s;
-    for (int i = tid; i < n_vocab; i += kSelThreads) {
-      const uint32_t key = order_key(l[i]);
-      if ((key & hmask) == prefix) atomicAdd(&hist[(key >> shift) & 0xFF], 1u);
-    }
-    __syncthreads();
-    if (tid == 0) {
-      uint32_t rem = remain_s, b = 255;
-      for (;; --b) {  // from the largest digit down: the bin that holds the rem-th largest key
-        if (hist[b] >= rem || b == 0) break;
-        rem -= hist[b];
+  __shared__ int taken[kSlices], again;
+  const int tid = threadIdx.x, r = blockIdx.x;
+  const int keep = slice_keep(k);
+  auto put = [&](uint32_t slot, uint32_t kk, int32_t ii) {
+    ckey[slot] = kk;
+    cidx[slot] = ii;
+  };
+  bool walk = cand == nullptr;
+  if (!walk) {
+    const int n = kSlices * keep;
+    const uint2* c = cand + (int64_t)r * n;
+    if (tid < kSlices) taken[tid] = 0;
+    if (tid == 0) again = 0;
+    auto from_cand = [&]<int M>() __attribute__((always_inline)) {
+      uint32_t key[M];
+      int32_t id[M];
+#pragma unroll
+      for (int e = 0; e < M; ++e) {
+        const int i = e * NT + tid;
+        const uint2 v = i < n ? c[i] : make_uint2(0u, (uint32_t)INT32_MAX);
+        key[e] = v.x;
+        id[e] = (int32_t)v.y;
       }
-      prefix_s = prefix | (b << shift);
-      remain_s = rem;
-    }
+      select_k(key, id, k, L, put);
+    };
+    if (n <= 2 * NT)
+      from_cand.template operator()<2>();
+    else
+      from_cand.template operator()<E>();
     __syncthreads();
-  }
-  const uint32_t T = prefix_s;
-  const uint32_t need_eq = remain_s;  // keys equal to T to take, lowest indices first
-  // Keys above T: exactly k - need_eq of them, in any order (sorted below).
-  if (tid == 0) count_s = 0;
-  __syncthreads();
-  for (int i = tid; i < n_vocab; i += kSelThreads) {
-    const uint32_t key = order_key(l[i]);
-    if (key > T) {
-      const uint32_t slot = atomicAdd(&count_s, 1u);
-      ckey[slot] = key;
-      cidx[slot] = i;
-    }
-  }
-  __syncthreads();
-  // Keys equal to T in index order: chunks of kSelThreads consecutive indices, ranked by a block prefix count.
-  uint32_t taken = 0;
-  const uint32_t base = (uint32_t)k - need_eq;
-  for (int c0 = 0; c0 < n_vocab && taken < need_eq; c0 += kSelThreads) {
-    const int i = c0 + tid;
-    const bool eq = i < n_vocab && order_key(l[i]) == T;
-    const unsigned long long bal = __ballot(eq);
-    const uint32_t lane = tid & 63, wave = tid >> 6;
-    if (lane == 0) scan[wave] = (uint32_t)__popcll(bal);
+    for (int i = tid; i < k; i += NT)
+      if (atomicAdd(&taken[(uint32_t)cidx[i] / kChunk % kSlices], 1) + 1 >= keep && keep < k) again = 1;
     __syncthreads();
-    uint32_t before = 0, total = 0;
-    for (int w = 0; w < kSelThreads / 64; ++w) {
-      before += w < (int)wave ? scan[w] : 0u;
-      total += scan[w];
-    }
-    const uint32_t rank = taken + before + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
-    if (eq && rank < need_eq) {
-      ckey[base + rank] = T;
-      cidx[base + rank] = i;
-    }
-    taken += total;
-    __syncthreads();
+    walk = again != 0;
   }
-  // Bitonic sort of the k candidates (padded to a power of two) by key descending, index ascending.
+  if (walk) {
+    const float* l = logits + (int64_t)(rows ? rows[r] : r) * stride;
+    uint32_t key[E];
+    int32_t id[E];
+    for (int pos = 0, held = 0; pos < n_vocab;) {
+      const int take = min(n_vocab - pos, E * NT - held);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int i = e * NT + tid, j = i - held;
+        const bool in = j >= 0 && j < take;
+        id[e] = in ? pos + j : i < held ? cidx[i] : INT32_MAX;
+        key[e] = in ? order_key(l[pos + j]) : i < held ? ckey[i] : 0u;
+      }
+      __syncthreads();  // the best so far have been read
+      select_k(key, id, k, L, put);
+      pos += take;
+      held = k;
+      __syncthreads();  // they have been written, L has been read
+    }
+  }
+  // Sorted by key descending, index ascending: up to 128 by counting those before each, more by a bitonic sort
+  // (padded to a power of two).
+  auto before_in_order = [](uint32_t ka, int ia, uint32_t kb, int ib) { return ka > kb || (ka == kb && ia < ib); };
+  auto emit = [&](int i, uint32_t u, int32_t ii) {  // order_key undone: the logit's own bits
+    out_i[(int64_t)r * k + i] = ii;
+    out_v[(int64_t)r * k + i] = __uint_as_float((u & 0x80000000u) ? u & 0x7FFFFFFFu : ~u);
+  };
+  if (k <= 128) {
+    __syncthreads();
+    if (tid < k) {
+      const uint32_t u = ckey[tid];
+      const int32_t ii = cidx[tid];
+      int rank = 0;
+      for (int j = 0; j < k; ++j) rank += before_in_order(ckey[j], cidx[j], u, ii) ? 1 : 0;
+      emit(rank, u, ii);
+    }
+    return;
+  }
   int n2 = 1;
   while (n2 < k) n2 <<= 1;
-  for (int i = k + tid; i < n2; i += kSelThreads) {
+  for (int i = k + tid; i < n2; i += NT) {
     ckey[i] = 0u;
-    cidx[i] = 0x7FFFFFFF;
+    cidx[i] = INT32_MAX;
   }
   __syncthreads();
-  auto before_in_order = [](uint32_t ka, int ia, uint32_t kb, int ib) { return ka > kb || (ka == kb && ia < ib); };
   for (int size = 2; size <= n2; size <<= 1)
     for (int stride2 = size >> 1; stride2 > 0; stride2 >>= 1) {
-      for (int i = tid; i < n2; i += kSelThreads) {
+      for (int i = tid; i < n2; i += NT) {
         const int j = i ^ stride2;
         if (j > i) {
           const bool up = (i & size) == 0;  // this run sorted in order (up) or reversed
@@ -141,10 +273,7 @@ __global__ __launch_bounds__(kSelThreads) void k_topk(const float* __restrict__ 
       }
       __syncthreads();
     }
-  for (int i = tid; i < k; i += kSelThreads) {
-    out_i[(int64_t)r * k + i] = cidx[i];
-    out_v[(int64_t)r * k + i] = l[cidx[i]];
-  }
+  for (int i = tid; i < k; i += NT) emit(i, ckey[i], cidx[i]);
 }
 
 }  // namespace
@@ -158,11 +287,29 @@ void penalize(hipStream_t s, float* logits, int64_t stride, const int32_t* rows,
   check_launch("penalize");
 }
 
+// Rows of up to kOneSlice logits take one workgroup each; longer ones kSlices slices, whose candidates go through the
+// scratch, as many rows per pair of launches as it holds (40 KB per row at k = 1024). Measured, with one
+// workgroup walking each row -> this form: 8 rows of 151936 at k = 40 267 -> 29.5 us (1024: 276 -> 55), one row
+// 203 -> 25, 64 rows 384 -> 115, 8 rows of 8193 60 -> 28; of 8192, which one workgroup selects from registers in one
+// round (slices would cost the second launch), 57 -> 17.
 void topk(hipStream_t s, const float* logits, int64_t stride, const int32_t* rows, int n_rows, int n_vocab, int k,
-          float* out_v, int32_t* out_i) {
+          float* out_v, int32_t* out_i, void* scratch, size_t scratch_bytes) {
   if (n_rows <= 0) return;
   require(k >= 1 && k <= kMaxTopK && k <= n_vocab, "topk: k must be 1..1024 and at most the vocabulary");
-  hipLaunchKernelGGL(k_topk, dim3(n_rows), dim3(kSelThreads), 0, s, logits, stride, rows, n_vocab, k, out_v, out_i);
+  const bool sliced = n_vocab > kOneSlice;
+  const int keep = slice_keep(k);
+  const int batch = sliced ? (int)std::min<size_t>(n_rows, scratch_bytes / (kSlices * keep * sizeof(uint2))) : n_rows;
+  require(batch > 0, "topk: scratch too small");
+  uint2* cand = sliced ? static_cast<uint2*>(scratch) : nullptr;
+  for (int r0 = 0; r0 < n_rows; r0 += batch) {
+    const int nr = std::min(batch, n_rows - r0);
+    const float* l = rows ? logits : logits + (int64_t)r0 * stride;
+    const int32_t* rr = rows ? rows + r0 : nullptr;
+    if (sliced)
+      hipLaunchKernelGGL(k_topk_part, dim3(kSlices, nr), dim3(kPartThreads), 0, s, l, stride, rr, n_vocab, keep, cand);
+    hipLaunchKernelGGL(k_topk_final, dim3(nr), dim3(kSelThreads), 0, s, l, stride, rr, n_vocab, cand, k,
+                       out_v + (int64_t)r0 * k, out_i + (int64_t)r0 * k);
+  }
   check_launch("topk");
 }
 

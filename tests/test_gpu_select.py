@@ -1,0 +1,33 @@
+"""mk_topk where its forms meet: rows that one workgroup takes alone (up to 8192 logits), rows cut into 64 slices, slices
+walked in rounds (more than 4096 logits each), rows whose largest logits fall into one slice (the row is then walked
+whole), and more rows than the context's scratch holds candidates for, against numpy's stable order."""
+import numpy as np
+import pytest
+
+import malkin_amd as mk_
+from test_gpu_sampling import expected_topk
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("V,k,n_rows", [(8192, 1024, 2), (8193, 257, 2), (8193, 1024, 5), (32 * 1024 + 5, 1, 2),
+                                        (64 * 4096, 300, 3), (64 * 4096 + 1, 300, 3), (64 * 4096 + 64, 1024, 3),
+                                        (1 << 20, 1000, 3), (20000, 128, 70), (20000, 129, 3), (151936, 1024, 30)])
+def test_topk_forms(mk, V, k, n_rows):
+    rng = np.random.default_rng(V + k)
+    x = rng.standard_normal((n_rows, V)).astype(np.float32)
+    x[0] = np.round(x[0] * 2) / 2      # ties across slices
+    if n_rows > 1:
+        x[1] = -np.inf                 # every logit equal and the lowest
+        x[1, V // 2] = np.float32(1.0)
+    if n_rows > 2:
+        x[2, np.arange(V) // 64 % 64 == 5] += 20.0  # the largest logits in one slice
+    dx = mk.to_device(x)
+    dv, di = mk.alloc(n_rows * k * 4), mk.alloc(n_rows * k * 4)
+    print("topk forms", V, k, n_rows, flush=True)
+    mk_.check(mk_.load().mk_topk(mk.h, dx.ptr, V, None, n_rows, V, k, dv.ptr, di.ptr))
+    gv, gi = dv.download(np.float32).reshape(n_rows, k), di.download(np.int32).reshape(n_rows, k)
+    for r in range(n_rows):
+        ev, ei = expected_topk(x[r], k)
+        assert np.array_equal(gi[r], ei), (V, k, r)
+        assert np.array_equal(gv[r].view(np.uint32), ev.view(np.uint32)), (V, k, r)
