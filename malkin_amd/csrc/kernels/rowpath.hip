@@ -7,8 +7,7 @@
 //   apart); lane 0 finishes the scalar parts (the F types' k % 16 tail, Q8_0's odd last block, the K-quants' mins /
 //   bias chains).
 // A wave holds four groups, a workgroup sixteen: one weight row per group, NT tokens of it at once so that a row is read
-// once per token tile. These weights are off the configurations' hot path (every matmul weight there is quantized and
-// packed); the kernel favours the reference's exact order over bandwidth.
+// once per token tile. F32 / F16 / BF16 rows go to the matrix cores instead (k_rows_mfma) unless they are unaligned.
 #include "ctx.h"
 #include "ops.h"
 
@@ -262,6 +261,248 @@ __global__ __launch_bounds__(kRowsThreads) void k_gguf45(const uint8_t* __restri
       }
 }
 
+// F32 / F16 / BF16 rows on the matrix cores. v_mfma_f32_16x16x4_f32 runs each output element as four fmas in
+// ascending k, each rounded once (measured bit for bit against fmaf over normal, denormal, infinite and signed-zero
+// operands), so one instruction advances a lane chain of kernels_avx512.cpp:82-107 by four steps for 16 rows x 16
+// tokens. Chain l takes elements 16 c + l: MFMA k index q is chunk c + q, so a lane that reads four consecutive values
+// of chunk c + lane / 16 holds the operands of four chains.
+//
+// A workgroup owns 16 RT rows by 16 TT tokens and walks K in stages of KS steps of 64 columns, held in a ring of NS LDS
+// buffers that direct global -> LDS copies fill NS - 1 stages ahead (16-byte pieces: lanes reading their operands
+// straight from global memory touch 64 separate 64-byte segments per load, which bound the kernel at 60 TFLOP/s).
+// Wave w runs chains 4 w .. 4 w + 3 of all the outputs; the halving tree then joins the waves' chains through LDS.
+// The pieces of a row are stored rotated (xor) so that the 16 rows of a read fall on different banks.
+// What bounds it: for prompts the fp32 matrix rate (153 TFLOP/s measured on a large product), for a few tokens the
+// stream of weights. Measured in
+// BF16, one 16-lane group per row with scalar loads (k_rows) -> this: 19456 x 2560 at 256 tokens 4858 -> 291 us, at one
+// 110 -> 23; 1024 x 3072 at 96 166 -> 14.
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+template <int TYPE>
+__device__ __forceinline__ void row_floats(const uint8_t* p, float (&v)[4]) {  // four consecutive weights
+  if constexpr (TYPE == kF32) {
+    const float4 f = *reinterpret_cast<const float4*>(p);
+    v[0] = f.x, v[1] = f.y, v[2] = f.z, v[3] = f.w;
+  } else {
+    const uint2 u = *reinterpret_cast<const uint2*>(p);
+    if constexpr (TYPE == kF16) {
+      v[0] = half_to_float((uint16_t)(u.x & 0xFFFF)), v[1] = half_to_float((uint16_t)(u.x >> 16));
+      v[2] = half_to_float((uint16_t)(u.y & 0xFFFF)), v[3] = half_to_float((uint16_t)(u.y >> 16));
+    } else {
+      v[0] = __uint_as_float(u.x << 16), v[1] = __uint_as_float(u.x & 0xFFFF0000u);
+      v[2] = __uint_as_float(u.y << 16), v[3] = __uint_as_float(u.y & 0xFFFF0000u);
+    }
+  }
+}
+template <int TYPE>
+__device__ __forceinline__ float row_value(const uint8_t* w, int64_t i) {
+  if constexpr (TYPE == kF32)
+    return reinterpret_cast<const float*>(w)[i];
+  else if constexpr (TYPE == kF16)
+    return half_to_float(reinterpret_cast<const uint16_t*>(w)[i]);
+  else
+    return bf16_to_float(reinterpret_cast<const uint16_t*>(w)[i]);
+}
+
+// TN: tokens staged per token tile (fewer than 16 for a few tokens; lanes past them repeat them, unused).
+template <int TYPE, int RT, int TT, int TN, int KS, int NS>
+struct RowTile {
+  static constexpr int elem = TYPE == kF32 ? 4 : 2;
+  static constexpr int wp = 64 * elem / 16;            // 16-byte pieces of a row per step
+  static constexpr int toks = TN * TT;
+  static constexpr int xpieces = toks * 16, pieces = xpieces + 16 * RT * wp;  // per step: x, then weights
+  static constexpr int loads = KS * pieces / 256;      // copies per wave and stage
+  static_assert(KS * pieces % 256 == 0 && xpieces % 64 == 0 && (TN == 16 || TT == 1), "whole copies per wave");
+  static constexpr int stage = KS * pieces * 16;       // bytes
+  static constexpr int part = 2 * 4 * RT * TT * 64 * 16;  // the tree's exchange, after the last stage
+  static constexpr int lds = NS * stage > part ? NS * stage : part;
+};
+
+template <int TYPE, int RT, int TT, int TN, int KS, int NS>
+__global__ __launch_bounds__(kRowsThreads) __attribute__((amdgpu_waves_per_eu(RT * TT == 4 ? 3 : 4))) void k_rows_mfma(const uint8_t* W, size_t row_bytes, int64_t rows,
+                                                            int64_t cols, const float* x, int64_t xs, int n,
+                                                            float* __restrict__ y, int64_t ys, int accumulate,
+                                                            int n_tt, int tiles) {
+  using T = RowTile<TYPE, RT, TT, TN, KS, NS>;
+  extern __shared__ __align__(16) uint8_t smem[];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15, q = lane >> 4;
+  const int tile = xcd_run((int)blockIdx.x, tiles);  // token tiles of a row tile on one XCD: its rows are read once
+  const int64_t r0 = (int64_t)(tile / n_tt) * (16 * RT);
+  const int t0 = (tile % n_tt) * (16 * TT);
+  const int chunks = (int)(cols / 16), nstages = (chunks + 4 * KS - 1) / (4 * KS);
+
+  // This lane's copies: piece g of the stage comes from chunk cc[j] of the stage (clamped to the last chunk), at
+  // src[j] plus whole chunks.
+  const uint8_t* src[T::loads];
+  int cc[T::loads];
+#pragma unroll
+  for (int j = 0; j < T::loads; ++j) {
+    const int g0 = (w * T::loads + j) * 64, ks = g0 / T::pieces, g = g0 % T::pieces + lane;
+    if (g0 % T::pieces < T::xpieces) {
+      const int tok = g / 16, p = (g % 16) ^ (tok & 15);
+      cc[j] = 4 * ks + p / 4;
+      src[j] = reinterpret_cast<const uint8_t*>(x + (int64_t)min(t0 + tok, n - 1) * xs) + 16 * (p % 4);
+    } else {
+      const int h = g - T::xpieces, row = h / T::wp;
+      const int p = (h % T::wp) ^ (T::wp == 16 ? row & 15 : (row >> 1) & 7);
+      constexpr int pc = T::wp / 4;  // pieces per chunk
+      cc[j] = 4 * ks + p / pc;
+      src[j] = W + (size_t)min(r0 + row, rows - 1) * row_bytes + 16 * (p % pc);
+    }
+  }
+  auto issue = [&](int st, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < T::loads; ++j) {
+      const int g0 = (w * T::loads + j) * 64;
+      const int bytes = g0 % T::pieces < T::xpieces ? 64 : 16 * T::elem;  // per chunk
+      lds_copy16(src[j] + (size_t)min(4 * KS * st + cc[j], chunks - 1) * bytes, smem + buf * T::stage + g0 * 16);
+    }
+  };
+  f4 acc[4][RT][TT];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int a = 0; a < RT; ++a)
+#pragma unroll
+      for (int b = 0; b < TT; ++b) acc[e][a][b] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto step = [&](const uint8_t* sp, int s) __attribute__((always_inline)) {
+    float wv[RT][4], xv[TT][4];
+#pragma unroll
+    for (int b = 0; b < TT; ++b) {
+      const int tok = 16 * b + i % TN;
+      const float4 f = *reinterpret_cast<const float4*>(sp + (tok * 16 + ((4 * q + w) ^ (tok & 15))) * 16);
+      xv[b][0] = f.x, xv[b][1] = f.y, xv[b][2] = f.z, xv[b][3] = f.w;
+    }
+#pragma unroll
+    for (int a = 0; a < RT; ++a) {
+      const int row = 16 * a + i;
+      const uint8_t* wr = sp + (T::xpieces + row * T::wp) * 16;
+      if constexpr (T::wp == 16)
+        row_floats<TYPE>(wr + ((4 * q + w) ^ (row & 15)) * 16, wv[a]);
+      else
+        row_floats<TYPE>(wr + ((2 * q + (w >> 1)) ^ ((row >> 1) & 7)) * 16 + 8 * (w & 1), wv[a]);
+    }
+    if (4 * s + 4 > chunks) {  // chunks past the last: fma(-0, 0, acc) == acc for every acc, -0 too
+      const bool in = 4 * s + q < chunks;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+#pragma unroll
+        for (int a = 0; a < RT; ++a) wv[a][e] = in ? wv[a][e] : 0.0f;
+#pragma unroll
+        for (int b = 0; b < TT; ++b) xv[b][e] = in ? xv[b][e] : -0.0f;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int a = 0; a < RT; ++a)
+#pragma unroll
+        for (int b = 0; b < TT; ++b)
+          acc[e][a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[b][e], wv[a][e], acc[e][a][b], 0, 0, 0);
+  };
+  for (int st = 0; st < NS - 1 && st < nstages; ++st) issue(st, st);
+  int buf = 0;
+  for (int st = 0; st < nstages; ++st) {
+    // Stage st has landed once at most the copies of the stages after it are outstanding; the buffer that stage
+    // st + NS - 1 goes into was read in stage st - 1, finished by every wave before this barrier.
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    wait_vm_stages<T::loads, NS - 2>(min(NS - 2, nstages - 1 - st));
+    ring_barrier();
+    if (st + NS - 1 < nstages) issue(st + NS - 1, buf == 0 ? NS - 1 : buf - 1);
+    const uint8_t* sp = smem + buf * T::stage;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) step(sp + ks * T::pieces * 16, KS * st + ks);
+    buf = buf == NS - 1 ? 0 : buf + 1;
+  }
+  __syncthreads();  // the ring becomes the tree's exchange
+  f4(*part)[4][RT * TT][64] = reinterpret_cast<f4(*)[4][RT * TT][64]>(smem);
+
+  // The halving tree over chains 4 w + e: pairs 8 apart are waves w and w + 2, pairs 4 apart waves 0 and 1, pairs 2 and
+  // 1 apart chains of one wave.
+  auto put = [&](int slot) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int a = 0; a < RT; ++a)
+#pragma unroll
+        for (int b = 0; b < TT; ++b) part[slot][e][a * TT + b][lane] = acc[e][a][b];
+  };
+  auto add = [&](int slot) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int a = 0; a < RT; ++a)
+#pragma unroll
+        for (int b = 0; b < TT; ++b) acc[e][a][b] = acc[e][a][b] + part[slot][e][a * TT + b][lane];
+  };
+  if (w >= 2) put(w - 2);
+  __syncthreads();
+  if (w < 2) add(w);
+  if (w == 1) put(1);  // this wave's own slot, which only it has read
+  __syncthreads();
+  if (w != 0) return;
+  add(1);
+#pragma unroll
+  for (int a = 0; a < RT; ++a)
+#pragma unroll
+    for (int b = 0; b < TT; ++b) {
+      const int64_t r = r0 + 16 * a + i;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int t = t0 + 16 * b + 4 * q + j;
+        if (r >= rows || t >= n) continue;
+        float v = (acc[0][a][b][j] + acc[2][a][b][j]) + (acc[1][a][b][j] + acc[3][a][b][j]);
+        for (int64_t k = 16 * (int64_t)chunks; k < cols; ++k)  // the scalar tail of k % 16 columns
+          v = fma_(row_value<TYPE>(W + (size_t)r * row_bytes, k), x[(int64_t)t * xs + k], v);
+        float* o = y + (int64_t)t * ys + r;
+        *o = accumulate ? *o + v : v;
+      }
+    }
+}
+
+// Tile rule: the largest tile that still gives the chip enough workgroups (a 32 x 32 tile runs at 75-88 TFLOP/s from
+// about four workgroups per CU, but at 12-30 below one). Measured in BF16, 16x16 / 16 rows x 32 tokens / 32x32, us:
+// 19456 x 2560 at 256 tokens 368 / 321 / 291 (4864 32 x 32 tiles), 6144 x 1024 at 96 22.6 / 21.3 / 22.6 (576), 2560 x 9728
+// at 96 72 / 67 / 67 (240; 480 tiles of 16 x 32), at 48 38 / 63 / 65 (160; 320), 1024 x 3072 at 96 14 / 16 / 23 (96).
+// Up to 4 tokens only 4 token rows are staged: 19456 x 2560 at one token 38 (16 rows staged) -> 23 us, 4.4 TB/s; with
+// no more workgroups than CUs stages twice as long (2560 x 9728: 21.9 -> 18.9 us).
+template <int TYPE>
+void launch_rows_mfma(hipStream_t s, const uint8_t* w, size_t row_bytes, int64_t rows, int64_t cols, const float* x,
+                      int64_t xs, int n, float* y, int64_t ys, bool accumulate) {
+  auto tiles = [&](int rt, int tt) { return (rows + 16 * rt - 1) / (16 * rt) * ((n + 16 * tt - 1) / (16 * tt)); };
+  auto go = [&]<int RT, int TT, int TN, int KS, int NS>() {
+    constexpr int lds = RowTile<TYPE, RT, TT, TN, KS, NS>::lds;
+    static_assert(lds <= 65536, "dynamic LDS without an attribute");
+    hipLaunchKernelGGL((k_rows_mfma<TYPE, RT, TT, TN, KS, NS>), dim3((unsigned)tiles(RT, TT)), dim3(kRowsThreads), lds, s,
+                       w, row_bytes, rows, cols, x, xs, n, y, ys, accumulate ? 1 : 0, (n + 16 * TT - 1) / (16 * TT),
+                       (int)tiles(RT, TT));
+  };
+  constexpr bool f32 = TYPE == kF32;
+  const int64_t cus = device_cus();
+  if (n <= 4) {
+    if (tiles(1, 1) > cus)
+      go.template operator()<1, 1, 4, 4, 2>();
+    else if constexpr (f32)
+      go.template operator()<1, 1, 4, 4, 3>();
+    else
+      go.template operator()<1, 1, 4, 8, 2>();
+  } else if (n > 16 && tiles(2, 2) >= 4 * cus) {
+    go.template operator()<2, 2, 16, 2, 2>();
+  } else if (n > 16 && 4 * tiles(1, 2) >= 7 * cus) {
+    go.template operator()<1, 2, 16, 2, 2>();
+  } else {
+    go.template operator()<1, 1, 16, 4, 2>();
+  }
+}
+
+// The MFMA form's copies: whole 16-byte pieces of aligned rows; at least one 16-value chunk.
+bool rows_mfma_ok(int type, const void* w, size_t row_bytes, int64_t rows, int64_t cols, const float* x, int64_t xs,
+                  int n) {
+  return (type == kF32 || type == kF16 || type == kBF16) && cols >= 16 && (uintptr_t)w % 16 == 0 &&
+         row_bytes % 16 == 0 && (uintptr_t)x % 16 == 0 && xs % 4 == 0 &&
+         (rows + 15) / 16 * ((n + 15) / 16) < INT32_MAX;
+}
+
 }  // namespace
 
 bool rows_supported(int type, int64_t cols) {
@@ -287,6 +528,17 @@ void matmul_rows(hipStream_t s, int type, const void* w, size_t row_bytes, int64
   if (rows <= 0 || n <= 0) return;
   const bool f = type == kF32 || type == kF16 || type == kBF16;
   require(f ? x != nullptr : xq != nullptr, "matmul_rows: missing activations (fp32 for F32/F16/BF16, BlockQ8 else)");
+  if (rows_mfma_ok(type, w, row_bytes, rows, cols, x, xs, n)) {
+    auto* wb = static_cast<const uint8_t*>(w);
+    if (type == kF32)
+      launch_rows_mfma<kF32>(s, wb, row_bytes, rows, cols, x, xs, n, y, ys, accumulate);
+    else if (type == kF16)
+      launch_rows_mfma<kF16>(s, wb, row_bytes, rows, cols, x, xs, n, y, ys, accumulate);
+    else
+      launch_rows_mfma<kBF16>(s, wb, row_bytes, rows, cols, x, xs, n, y, ys, accumulate);
+    check_launch("matmul_rows");
+    return;
+  }
   const dim3 grid((unsigned)((rows + kRowsThreads / 16 - 1) / (kRowsThreads / 16)), (unsigned)((n + kRowsNT - 1) / kRowsNT));
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(kRowsThreads), 0, s, static_cast<const uint8_t*>(w), row_bytes, rows, cols, x,
