@@ -16,6 +16,12 @@
 // layout.h into int8 in registers: Q4_K nibbles 0..15; Q6_K q - 32 per byte as ((q | 0x80) - 0x20) ^ 0x80, which
 // never borrows across bytes for q < 64.
 //
+// What bounds it: one wave per SIMD is a serial chain of LDS reads, an MFMA, its conversion and 32 (Q4_K) or 48 (Q6_K wide)
+// vector fmas per unit, about 600 cycles where the fmas alone take 130-190. So a unit's dots and products are issued
+// on the matrix pipe while the unit before it runs its epilogue on the vector pipe, its operands are read one unit
+// ahead, and a stage's last unit finishes in the next stage. Q4_K 2560 x 9728 at 203 tokens 86 -> 70 us, 5120 x 17408 at
+// 100 150 -> 122; Q6_K 2560 x 9728 at 203 96 -> 86, 19456 x 2560 at 512 200 -> 187, 34816 x 5120 at 17 60 -> 58.
+//
 // A workgroup (4 waves) owns a 128-row x 32-token tile (or a 32-row tail tile), 32 rows per wave, and walks K in
 // stages of half a super-block (4 units of 32 weights) held in a ring of NS LDS buffers filled by direct global -> LDS
 // loads NS - 1 stages ahead.
@@ -106,6 +112,9 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
                                                       const BlockQ8* x, int n, float* __restrict__ y, int64_t ys,
                                                       int accumulate, int n_rt, int n_tt, int n_big) {
   using S = KqLds<TYPE>;
+  // Q4_K on large grids runs three waves per SIMD, which cover each other's latency; the pipeline's second register set
+  // would leave two (19456 x 2560 at 512 tokens 135 us without it, 144 with it; 5120 x 17408 268 and 286).
+  constexpr bool kPipe = !(TYPE == kQ4_K && NS == 3);
   extern __shared__ __align__(16) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wu = __builtin_amdgcn_readfirstlane(w);
@@ -247,6 +256,46 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
     return v;
   };
 
+  // One unit in the pipeline: its MFMA results and the operands of its epilogue. Q4_K: f0 = float(dot), p2 (below), b =
+  // dx (s0 + s1) per token, s0 = -(dmin m). Q6_K: f0 / f1 = the halves' float(dot); wide: b = dx per token, s0 / s1 = d
+  // sc of the halves; compact: p = (d sc_h) dx, halves 0 and 1.
+  struct Unit {
+    v16f f0, f1, b;
+    v32f p;
+    float s0 = 0.0f, s1 = 0.0f;
+  };
+  Unit U[2];
+  v16i i0 = magic, i1 = magic;  // the next unit's int dots, between its two steps
+  v32f p2 = zero;               // Q4_K: (d sc_j) dx of the unit pair
+  U[1].f0 = U[1].f1 = U[1].b = v16f{};
+  U[1].p = v32f{};
+
+  // The first and second half of a unit's epilogue, in the reference's order.
+  auto epi_a = [&](const Unit& u, int odd) __attribute__((always_inline)) {
+    if constexpr (TYPE == kQ6_K && WIDE) {
+#pragma unroll
+      for (int i = 0; i < NE / 2; ++i) acc[i] = fma_(fma_(u.f1[i], u.s1, u.f0[i] * u.s0), u.b[i], acc[i]);
+    } else if constexpr (TYPE == kQ6_K) {
+#pragma unroll
+      for (int i = 0; i < NE; ++i) acc[i] = fma_(u.f0[i], u.p[i], acc[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NE; ++i) acc[i] = fma_(u.f0[i], p2[16 * odd + i], acc[i]);
+    }
+  };
+  auto epi_b = [&](const Unit& u) __attribute__((always_inline)) {
+    if constexpr (TYPE == kQ6_K && WIDE) {
+#pragma unroll
+      for (int i = NE / 2; i < NE; ++i) acc[i] = fma_(fma_(u.f1[i], u.s1, u.f0[i] * u.s0), u.b[i], acc[i]);
+    } else if constexpr (TYPE == kQ6_K) {
+#pragma unroll
+      for (int i = 0; i < NE; ++i) acc[i] = fma_(u.f1[i], u.p[16 + i], acc[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NE; ++i) acc[i] = fma_(u.s0, u.b[i], acc[i]);
+    }
+  };
+
   auto stage = [&]<int BUF, bool TAIL>(int s) __attribute__((always_inline)) {
     // Stage s has landed once at most the loads of the stages issued after it (s + 1 .. s + NS - 2, fewer at the
     // end) are outstanding; the buffer stage s + NS - 1 goes into was read in stage s - 1, finished by every wave
@@ -261,47 +310,18 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
     if (!live) return;
     uint8_t* st = smem + BUF * S::bytes;
     const int hf = s & 1;
+    // The lane's weight scales for the stage, then per unit: `begin` reads its operands and issues the int dots,
+    // `mid` converts them and issues the scale products.
+    float sca[kKB], scb[kKB];
+    uint4 raw[2];
     if constexpr (TYPE == kQ6_K) {
-      // weight scales of this lane's row: d, and sc_h for the 8 halves of units 4 hf .. 4 hf + 3
       const float d = half_to_float(*reinterpret_cast<const uint16_t*>(st + S::d + gi * 16 + r8 * 2));
       const uint2 scw = *reinterpret_cast<const uint2*>(st + S::sc + gi * 128 + r8 * 16 + 8 * hf);
 #pragma unroll
       for (int u = 0; u < kKB; ++u) {
         const uint32_t sw = u < 2 ? scw.x : scw.y;
-        const float d0 = d * sbyte_f<0>(sw >> (16 * (u & 1))), d1 = d * sbyte_f<1>(sw >> (16 * (u & 1)));
-        const uint8_t* au = st + S::a + u * 3072 + gi * 192;
-        const uint2 nib = *reinterpret_cast<const uint2*>(au + r8 * 16 + 8 * h);
-        const uint2 hb = *reinterpret_cast<const uint2*>(au + 128 + r8 * 8);
-        const uint8_t* xu = st + S::x + u * 1024 + li * 32 + 8 * h;
-        const long xa0 = *reinterpret_cast<const long*>(xu), xa1 = *reinterpret_cast<const long*>(xu + 16);
-        // half hw: bytes r = 0..7 are q[16 hw + 8 h + r]
-        long wq[2];
-#pragma unroll
-        for (int hw = 0; hw < 2; ++hw) {
-          const uint32_t hv = (hw ? hb.y : hb.x) >> (4 * h);
-          const uint32_t q0 = ((nib.x >> (4 * hw)) & 0x0F0F0F0Fu) | ((hv & 0x03030303u) << 4);
-          const uint32_t q1 = ((nib.y >> (4 * hw)) & 0x0F0F0F0Fu) | (((hv >> 2) & 0x03030303u) << 4);
-          wq[hw] = (long)(((uint64_t)minus32(q1) << 32) | minus32(q0));
-        }
-        const v16f f0 = conv(__builtin_amdgcn_mfma_i32_32x32x16_i8(xa0, wq[0], magic, 0, 0, 0));
-        const v16f f1 = conv(__builtin_amdgcn_mfma_i32_32x32x16_i8(xa1, wq[1], magic, 0, 0, 0));
-        if constexpr (WIDE) {
-          const v16f dx = tok16(st + S::dx + u * 128);
-#pragma unroll
-          for (int i = 0; i < NE; ++i) {
-            const float sm = fma_(f1[i], d1, f0[i] * d0);
-            acc[i] = fma_(sm, dx[i], acc[i]);
-          }
-        } else {
-          // (d sc_h) dx for both halves: block h of the outer product takes dx (A) and d sc_h (B)
-          const float dxl = *reinterpret_cast<const float*>(st + S::dx + u * 128 + li * 4);
-          const v32f p = __builtin_amdgcn_mfma_f32_32x32x1f32(dxl, h ? d1 : d0, zero, 0, 0, 0);
-#pragma unroll
-          for (int i = 0; i < NE; ++i) {
-            acc[i] = fma_(f0[i], p[i], acc[i]);
-            acc[i] = fma_(f1[i], p[16 + i], acc[i]);
-          }
-        }
+        sca[u] = d * sbyte_f<0>(sw >> (16 * (u & 1)));
+        scb[u] = d * sbyte_f<1>(sw >> (16 * (u & 1)));
       }
     } else {
       // dx (s0 + s1) of the stage's 4 units x 32 tokens, into this wave's own copy
@@ -313,40 +333,133 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
         const int ss = (int)(int16_t)(sv & 0xFFFF) + (int)(int16_t)(sv >> 16);
         *reinterpret_cast<float*>(st + S::dsx + w * 512 + 4 * p) = dxv * (float)ss;
       }
+#pragma unroll
+      for (int cc = 0; cc < 2; ++cc)
+        raw[cc] = *reinterpret_cast<const uint4*>(st + S::a + cc * 4096 + gi * 256 + h * 128 + r8 * 16);
       const uint4 hd = *reinterpret_cast<const uint4*>(st + S::hdr + gi * 128 + r8 * 16);
       const float d = half_to_float((uint16_t)(hd.x & 0xFFFF)), dmin = half_to_float((uint16_t)(hd.x >> 16));
-      float fsc[kKB], fmn[kKB];
+      // scale_min_k4 of sub-blocks 4 hf + 0..3, byte u of each word (hd.y, hd.z, hd.w: the 12 packed bytes): the low
+      // half of a super-block takes 6 bits of hd.y / hd.z, the high half nibbles of hd.w and the top bits of those.
+      const uint32_t sc4 = hf ? (hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u) : hd.y & 0x3F3F3F3Fu;
+      const uint32_t mn4 = hf ? ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u) : hd.z & 0x3F3F3F3Fu;
 #pragma unroll
       for (int u = 0; u < kKB; ++u) {
-        int sc, m;
-        scale_min(4 * hf + u, hd.y, hd.z, hd.w, sc, m);
-        fsc[u] = d * (float)sc;
-        fmn[u] = dmin * (float)m;
+        sca[u] = d * (float)((sc4 >> (8 * u)) & 0xFFu);
+        scb[u] = -(dmin * (float)((mn4 >> (8 * u)) & 0xFFu));
       }
+    }
+    if constexpr (!kPipe) {
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc) {
-        const uint4 raw = *reinterpret_cast<const uint4*>(st + S::a + cc * 4096 + gi * 256 + h * 128 + r8 * 16);
         // (d sc_j) dx for units 2 cc and 2 cc + 1: block h takes unit 2 cc + h
         const float dxl = *reinterpret_cast<const float*>(st + S::dx + (2 * cc + h) * 128 + li * 4);
-        const v32f p = __builtin_amdgcn_mfma_f32_32x32x1f32(dxl, h ? fsc[2 * cc + 1] : fsc[2 * cc], zero, 0, 0, 0);
+        const v32f p = __builtin_amdgcn_mfma_f32_32x32x1f32(dxl, h ? sca[2 * cc + 1] : sca[2 * cc], zero, 0, 0, 0);
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           const int u = 2 * cc + e;
-          const v4i wq = e ? v4i{(int)((raw.x >> 4) & 0x0F0F0F0Fu), (int)((raw.y >> 4) & 0x0F0F0F0Fu),
-                                 (int)((raw.z >> 4) & 0x0F0F0F0Fu), (int)((raw.w >> 4) & 0x0F0F0F0Fu)}
-                           : v4i{(int)(raw.x & 0x0F0F0F0Fu), (int)(raw.y & 0x0F0F0F0Fu), (int)(raw.z & 0x0F0F0F0Fu),
-                                 (int)(raw.w & 0x0F0F0F0Fu)};
+          const v4i wq = {(int)((raw[cc].x >> (4 * e)) & 0x0F0F0F0Fu), (int)((raw[cc].y >> (4 * e)) & 0x0F0F0F0Fu),
+                          (int)((raw[cc].z >> (4 * e)) & 0x0F0F0F0Fu), (int)((raw[cc].w >> (4 * e)) & 0x0F0F0F0Fu)};
           const v4i xa = *reinterpret_cast<const v4i*>(st + S::x + u * 1024 + li * 32 + 16 * h);
           const v16f f = conv(__builtin_amdgcn_mfma_i32_32x32x32_i8(xa, wq, magic, 0, 0, 0));
           const v16f dsx = tok16(st + S::dsx + w * 512 + u * 128);
-          const float nm = -fmn[u];
 #pragma unroll
           for (int i = 0; i < NE; ++i) {
             acc[i] = fma_(f[i], p[16 * e + i], acc[i]);
-            acc[i] = fma_(nm, dsx[i], acc[i]);
+            acc[i] = fma_(scb[u], dsx[i], acc[i]);
           }
         }
       }
+      return;
+    }
+    // A unit's operands, read one unit ahead of its dots (Q4_K: x; Q6_K: nibbles, high bits, the halves of x).
+    struct Ops {
+      v4i xa;
+      uint2 nib, hb;
+      long xa0, xa1;
+    } ops[2];
+    auto read = [&](int u) __attribute__((always_inline)) {
+      Ops& o = ops[u & 1];
+      if constexpr (TYPE == kQ6_K) {
+        const uint8_t* au = st + S::a + u * 3072 + gi * 192;
+        o.nib = *reinterpret_cast<const uint2*>(au + r8 * 16 + 8 * h);
+        o.hb = *reinterpret_cast<const uint2*>(au + 128 + r8 * 8);
+        const uint8_t* xu = st + S::x + u * 1024 + li * 32 + 8 * h;
+        o.xa0 = *reinterpret_cast<const long*>(xu);
+        o.xa1 = *reinterpret_cast<const long*>(xu + 16);
+      } else {
+        o.xa = *reinterpret_cast<const v4i*>(st + S::x + u * 1024 + li * 32 + 16 * h);
+      }
+    };
+    // The unit's int dots; its per-token operands are read behind them.
+    float dxl = 0.0f;
+    auto begin = [&](Unit& n, int u) __attribute__((always_inline)) {
+      const Ops& o = ops[u & 1];
+      if constexpr (TYPE == kQ6_K) {
+        // half hw: bytes r = 0..7 are q[16 hw + 8 h + r]
+        long wq[2];
+#pragma unroll
+        for (int hw = 0; hw < 2; ++hw) {
+          const uint32_t hv = (hw ? o.hb.y : o.hb.x) >> (4 * h);
+          const uint32_t q0 = ((o.nib.x >> (4 * hw)) & 0x0F0F0F0Fu) | ((hv & 0x03030303u) << 4);
+          const uint32_t q1 = ((o.nib.y >> (4 * hw)) & 0x0F0F0F0Fu) | (((hv >> 2) & 0x03030303u) << 4);
+          wq[hw] = (long)(((uint64_t)minus32(q1) << 32) | minus32(q0));
+        }
+        i0 = __builtin_amdgcn_mfma_i32_32x32x16_i8(o.xa0, wq[0], magic, 0, 0, 0);
+        i1 = __builtin_amdgcn_mfma_i32_32x32x16_i8(o.xa1, wq[1], magic, 0, 0, 0);
+        if constexpr (WIDE)
+          n.b = tok16(st + S::dx + u * 128);
+        else
+          dxl = *reinterpret_cast<const float*>(st + S::dx + u * 128 + li * 4);
+      } else {
+        const uint4 r = raw[u >> 1];
+        const int sh = 4 * (u & 1);
+        const v4i wq = {(int)((r.x >> sh) & 0x0F0F0F0Fu), (int)((r.y >> sh) & 0x0F0F0F0Fu),
+                        (int)((r.z >> sh) & 0x0F0F0F0Fu), (int)((r.w >> sh) & 0x0F0F0F0Fu)};
+        i0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.xa, wq, magic, 0, 0, 0);
+        n.b = tok16(st + S::dsx + w * 512 + u * 128);
+        if (u % 2 == 0) dxl = *reinterpret_cast<const float*>(st + S::dx + (u + h) * 128 + li * 4);
+      }
+      if (u + 1 < kKB) read(u + 1);
+    };
+    // Its float dots and scale products.
+    auto mid = [&](Unit& n, int u) __attribute__((always_inline)) {
+      n.f0 = conv(i0);
+      if constexpr (TYPE == kQ6_K) {
+        n.f1 = conv(i1);
+        n.s0 = sca[u];
+        n.s1 = scb[u];
+        // compact: (d sc_h) dx for both halves: block h of the outer product takes dx (A) and d sc_h (B)
+        if constexpr (!WIDE) n.p = __builtin_amdgcn_mfma_f32_32x32x1f32(dxl, h ? scb[u] : sca[u], zero, 0, 0, 0);
+      } else {
+        n.s0 = scb[u];
+        // (d sc_j) dx for units u and u + 1: block h takes unit u + h
+        if (u % 2 == 0) p2 = __builtin_amdgcn_mfma_f32_32x32x1f32(dxl, h ? sca[u + 1] : sca[u], zero, 0, 0, 0);
+      }
+    };
+    // While a unit's epilogue runs on the vector pipe, the next unit's dots and products run on the matrix pipe; the
+    // stage's last unit finishes in the next stage (whose first operands are read behind its epilogue's first half).
+    // The scheduling barriers keep the two interleaved.
+    read(0);
+    __builtin_amdgcn_sched_barrier(0);
+    epi_a(U[1], 1);
+    __builtin_amdgcn_sched_barrier(0);
+    begin(U[0], 0);
+    __builtin_amdgcn_sched_barrier(0);
+    epi_b(U[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    mid(U[0], 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 1; u < kKB; ++u) {
+      Unit &cur = U[(u + 1) & 1], &nxt = U[u & 1];
+      begin(nxt, u);
+      __builtin_amdgcn_sched_barrier(0);
+      epi_a(cur, (u + 1) & 1);
+      __builtin_amdgcn_sched_barrier(0);
+      mid(nxt, u);
+      __builtin_amdgcn_sched_barrier(0);
+      epi_b(cur);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
@@ -371,6 +484,10 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
 
   // Element i: token t0 + 8 (i / 4) + 4 h + i % 4, row 128 rt + 32 w + li.
   if (live) {
+    if constexpr (kPipe) {
+      epi_a(U[1], 1);
+      epi_b(U[1]);
+    }
     float* yr = y + r0 + 32 * w + li;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
