@@ -1,5 +1,5 @@
-// Prefill / batch GEMM for K-quant weights (Q4_K, Q6_K) on int8 MFMA, bit-identical to the reference's panel kernels:
-//   Q4_K (gemm_avx512.cpp:104-155, the wide panels use the same arithmetic), per 32-weight sub-block j in order:
+// Prefill / batch GEMM for K-quant weights (Q4_K, Q6_K, and Q5_K from its GGUF rows) on int8 MFMA, bit-identical to the reference's panel kernels:
+//   Q4_K, Q5_K (gemm_avx512.cpp:104-155, the wide panels use the same arithmetic), per 32-weight sub-block j in order:
 //     acc = fma(float(sum q4 x), (d sc_j) dx, acc);  acc = fma(-(dmin m_j), dx (s0 + s1), acc)
 //   Q6_K compact (gemm_avx512.cpp:157-205), per 16-value half h in order:
 //     acc = fma(float(sum (q6 - 32) x), (d sc_h) dx, acc)
@@ -71,6 +71,21 @@ struct KqLds<kQ4_K> {
   static constexpr int loads = 5;
 };
 
+// Q5_K rows stay GGUF rows (mk_matmul_gguf): per row of a stage 7 pieces of 16 bytes, the header (d, dmin, scales), the
+// super-block's 32 high-bit bytes and the half's 64 nibble bytes, in consecutive lanes' copies (whole 48- and 64-byte
+// runs of a row) and in LDS row after row: a 112-byte row stride puts 16 rows' pieces on different banks.
+template <>
+struct KqLds<kQ5_K> {
+  static constexpr int piece = 7;
+  static constexpr int a = 0;                         // [4 waves][32 rows][7][16 B], 4096 B per wave
+  static constexpr int x = a + 4 * 4096;              // [4 units][32 tok][32 B]
+  static constexpr int dx = x + 4 * 32 * 32;          // [4 units][32 tok] f32
+  static constexpr int s = dx + 4 * 32 * 4;           // [4 units][32 tok] int16 pair (s0, s1)
+  static constexpr int dsx = s + 4 * 32 * 4;          // [4 waves][4 units][32 tok] f32
+  static constexpr int bytes = dsx + 4 * 4 * 32 * 4;  // 23552
+  static constexpr int loads = 6;
+};
+
 __device__ __forceinline__ void load_lds16(const void* g, uint8_t* l) { lds_copy16(g, l); }
 __device__ __forceinline__ void load_lds4(const void* g, uint8_t* l) { lds_copy4(g, l); }
 // float(int8 byte K of v)
@@ -110,7 +125,7 @@ __device__ __forceinline__ void scale_min(int j, uint32_t q0, uint32_t q1, uint3
 template <int TYPE, bool WIDE, int NS, int NE>
 __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t rows, int64_t cols,
                                                       const BlockQ8* x, int n, float* __restrict__ y, int64_t ys,
-                                                      int accumulate, int n_rt, int n_tt, int n_big) {
+                                                      int accumulate, int n_rt, int n_tt, int n_big, size_t row_bytes) {
   using S = KqLds<TYPE>;
   // Q4_K on large grids runs three waves per SIMD, which cover each other's latency; the pipeline's second register set
   // would leave two (19456 x 2560 at 512 tokens 135 us without it, 144 with it; 5120 x 17408 268 and 286).
@@ -128,7 +143,8 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
   const int64_t r0 = rt < n_big ? (int64_t)rt * kRowsT : (int64_t)n_big * kRowsT + (int64_t)(rt - n_big) * 32;
   const int64_t g0 = r0 / 8;
   const int ngroups = (int)min<int64_t>(rt < n_big ? kRowsT / 8 : 4, rows / 8 - g0);  // 4 .. 16 (rows % 32 == 0)
-  const bool live = 32 * wu < 8 * ngroups;  // this wave's 32 rows hold a row of the matrix (else: copies only)
+  // this wave's 32 rows hold a row of the matrix (else: copies only)
+  const bool live = TYPE == kQ5_K ? r0 + 32 * wu < rows : 32 * wu < 8 * ngroups;
   const int t0 = tt * kTokT;
   const int nstages = nb / kKB;  // cols % 256 == 0: whole stages
 
@@ -140,8 +156,10 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
   const uint32_t tw_off = (uint32_t)(tw * nb * 40 + (lane >> 5) * 40);  // + 80 c for unit 2 c + lane / 32
 
   // Weight copies: every piece is 16 (or 4) bytes of a packed (group, unit) record, LDS destinations lane-linear.
-  uint32_t a_off[3], m_off, t_off = 0;
-  const uint8_t *a_base, *m_base, *d_base = nullptr;
+  uint32_t a_off[3], m_off = 0, t_off = 0;
+  const uint8_t *a_base = W, *m_base = nullptr, *d_base = nullptr;
+  const uint8_t* q_src[4];  // Q5_K: this lane's four pieces, at super-block 0 and half 0
+  uint32_t q_half[4];       // and their step to half 1
   uint32_t d_off = 0;
   if constexpr (TYPE == kQ6_K) {
     const PackedQ6_K L{rows, nsb};
@@ -162,6 +180,13 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
     // Tail tile (4 groups): wave w copies unit w of the stage, lanes 0..47 its 4 x 12 pieces; lanes 48..63 re-read
     // group 3 into the unused group 4-5 slots.
     t_off = (uint32_t)((min(lane / 12, ngroups - 1) * nsb * 8 + w) * 192 + 16 * (lane % 12));
+  } else if constexpr (TYPE == kQ5_K) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int g = min(64 * c + lane, 32 * S::piece - 1), p = g % S::piece;
+      q_src[c] = W + (size_t)min(r0 + 32 * w + g / S::piece, rows - 1) * row_bytes + 16 * p;
+      q_half[c] = p < 3 ? 0u : 64u;
+    }
   } else {
     const PackedQ4_K L{rows, nsb};
 #pragma unroll
@@ -217,6 +242,12 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
       }
       load_lds16(xb + (size_t)wu * 40 + x_off, st + S::x + 1024 * wu);
       if (wu != 3) load_lds16(xb + (size_t)wu * 40 + x_off, st + S::x + 1024 * wu);
+    } else if constexpr (TYPE == kQ5_K) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        load_lds16(q_src[c] + (size_t)sb * 176 + (hf ? q_half[c] : 0u), st + S::a + 4096 * wu + 1024 * c);
+      load_lds4(xb + 4 * (wu >> 1) + 80 * (wu & 1) + tw_off, st + (wu < 2 ? S::dx : S::s) + 256 * (wu & 1));
+      load_lds16(xb + (size_t)wu * 40 + x_off, st + S::x + 1024 * wu);
     } else {
       const uint8_t* ab = a_base + ((size_t)sb * 4 + 2 * hf) * 256;
 #pragma unroll
@@ -313,7 +344,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
     // The lane's weight scales for the stage, then per unit: `begin` reads its operands and issues the int dots,
     // `mid` converts them and issues the scale products.
     float sca[kKB], scb[kKB];
-    uint4 raw[2];
+    uint4 raw[2], qh;
     if constexpr (TYPE == kQ6_K) {
       const float d = half_to_float(*reinterpret_cast<const uint16_t*>(st + S::d + gi * 16 + r8 * 2));
       const uint2 scw = *reinterpret_cast<const uint2*>(st + S::sc + gi * 128 + r8 * 16 + 8 * hf);
@@ -333,10 +364,19 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
         const int ss = (int)(int16_t)(sv & 0xFFFF) + (int)(int16_t)(sv >> 16);
         *reinterpret_cast<float*>(st + S::dsx + w * 512 + 4 * p) = dxv * (float)ss;
       }
+      uint4 hd;
+      if constexpr (TYPE == kQ5_K) {
+        const uint8_t* row = st + S::a + 4096 * w + 16 * S::piece * li;
+        hd = *reinterpret_cast<const uint4*>(row);
+        qh = *reinterpret_cast<const uint4*>(row + 16 + 16 * h);
 #pragma unroll
-      for (int cc = 0; cc < 2; ++cc)
-        raw[cc] = *reinterpret_cast<const uint4*>(st + S::a + cc * 4096 + gi * 256 + h * 128 + r8 * 16);
-      const uint4 hd = *reinterpret_cast<const uint4*>(st + S::hdr + gi * 128 + r8 * 16);
+        for (int cc = 0; cc < 2; ++cc) raw[cc] = *reinterpret_cast<const uint4*>(row + 48 + 32 * cc + 16 * h);
+      } else {
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc)
+          raw[cc] = *reinterpret_cast<const uint4*>(st + S::a + cc * 4096 + gi * 256 + h * 128 + r8 * 16);
+        hd = *reinterpret_cast<const uint4*>(st + S::hdr + gi * 128 + r8 * 16);
+      }
       const float d = half_to_float((uint16_t)(hd.x & 0xFFFF)), dmin = half_to_float((uint16_t)(hd.x >> 16));
       // scale_min_k4 of sub-blocks 4 hf + 0..3, byte u of each word (hd.y, hd.z, hd.w: the 12 packed bytes): the low
       // half of a super-block takes 6 bits of hd.y / hd.z, the high half nibbles of hd.w and the top bits of those.
@@ -413,8 +453,13 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
       } else {
         const uint4 r = raw[u >> 1];
         const int sh = 4 * (u & 1);
-        const v4i wq = {(int)((r.x >> sh) & 0x0F0F0F0Fu), (int)((r.y >> sh) & 0x0F0F0F0Fu),
-                        (int)((r.z >> sh) & 0x0F0F0F0Fu), (int)((r.w >> sh) & 0x0F0F0F0Fu)};
+        v4i wq = {(int)((r.x >> sh) & 0x0F0F0F0Fu), (int)((r.y >> sh) & 0x0F0F0F0Fu),
+                  (int)((r.z >> sh) & 0x0F0F0F0Fu), (int)((r.w >> sh) & 0x0F0F0F0Fu)};
+        if constexpr (TYPE == kQ5_K) {
+          const int j = 4 * hf + u;  // the sub-block's bit of the high-bit bytes
+          wq |= v4i{(int)(((qh.x >> j) & 0x01010101u) << 4), (int)(((qh.y >> j) & 0x01010101u) << 4),
+                    (int)(((qh.z >> j) & 0x01010101u) << 4), (int)(((qh.w >> j) & 0x01010101u) << 4)};
+        }
         i0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.xa, wq, magic, 0, 0, 0);
         n.b = tok16(st + S::dsx + w * 512 + u * 128);
         if (u % 2 == 0) dxl = *reinterpret_cast<const float*>(st + S::dx + (u + h) * 128 + li * 4);
@@ -492,7 +537,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int t = t0 + 8 * (i / 4) + tok_i + i % 4;
-      if (t < n) {
+      if (t < n && (TYPE != kQ5_K || r0 + 32 * w + li < rows)) {
         float* o = yr + (int64_t)t * ys;
         *o = accumulate ? *o + acc[i] : acc[i];
       }
@@ -502,7 +547,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
 
 template <int TYPE, bool WIDE, int NS, int NE>
 void launch_kq_ns(hipStream_t s, const void* w, int64_t rows, int64_t cols, const BlockQ8* x, int n, float* y,
-                  int64_t ys, bool accumulate, int n_rt, int n_tt, int n_big) {
+                  int64_t ys, bool accumulate, int n_rt, int n_tt, int n_big, size_t row_bytes = 0) {
   const size_t lds = NS * (size_t)KqLds<TYPE>::bytes;
   static bool attr = false;  // per instantiation: rings past 64 KB of dynamic LDS
   if (!attr) {
@@ -512,7 +557,8 @@ void launch_kq_ns(hipStream_t s, const void* w, int64_t rows, int64_t cols, cons
     attr = true;
   }
   hipLaunchKernelGGL((k_gemm_kq<TYPE, WIDE, NS, NE>), dim3((unsigned)((int64_t)n_rt * n_tt)), dim3(kThreads), lds, s,
-                     static_cast<const uint8_t*>(w), rows, cols, x, n, y, ys, accumulate ? 1 : 0, n_rt, n_tt, n_big);
+                     static_cast<const uint8_t*>(w), rows, cols, x, n, y, ys, accumulate ? 1 : 0, n_rt, n_tt, n_big,
+                     row_bytes);
 }
 
 // Ring depth by grid size: one workgroup per CU takes an 8-stage ring (7 stages, about 130 KB, in flight), two per CU
@@ -543,7 +589,35 @@ void launch_kq(hipStream_t s, const void* w, int64_t rows, int64_t cols, const B
     launch_kq_ns<TYPE, WIDE, 3, 16>(s, w, rows, cols, x, n, y, ys, accumulate, n_rt, n_tt, n_big);
 }
 
+// Q5_K: rings of 6 stages (138 KB) where the grid fits the CUs once, 3 (two workgroups per CU) past that; elements of
+// tokens past n are skipped in whole quarters (element i holds tokens 8 (i / 4) + 0..7). Measured against the
+// byte-wise kernel of rowpath.hip: 19456 x 2560 at 32 tokens 382 -> 23 us, at 256 2252 -> 87; 2560 x 9728 at 128 769 -> 72.
+void launch_q5(hipStream_t s, const void* w, size_t row_bytes, int64_t rows, int64_t cols, const BlockQ8* x, int n,
+               float* y, int64_t ys, bool accumulate) {
+  const int n_rt = (int)((rows + kRowsT - 1) / kRowsT), n_tt = (n + kTokT - 1) / kTokT;
+  auto go = [&]<int NE>() {
+    if ((int64_t)n_rt * n_tt <= device_cus())
+      launch_kq_ns<kQ5_K, false, 6, NE>(s, w, rows, cols, x, n, y, ys, accumulate, n_rt, n_tt, n_rt, row_bytes);
+    else
+      launch_kq_ns<kQ5_K, false, 3, NE>(s, w, rows, cols, x, n, y, ys, accumulate, n_rt, n_tt, n_rt, row_bytes);
+  };
+  if (n <= 8)
+    go.template operator()<4>();
+  else if (n <= 16)
+    go.template operator()<8>();
+  else
+    go.template operator()<16>();
+}
+
 }  // namespace
+
+void gemm_q5_gguf(hipStream_t s, const void* w, size_t row_bytes, int64_t rows, int64_t cols, const BlockQ8* x, int n,
+                  float* y, int64_t ys, bool accumulate) {
+  require(cols % 256 == 0 && rows > 0 && n > 0 && row_bytes % 16 == 0 && (uintptr_t)w % 16 == 0,
+          "gemm_q5_gguf: 16-byte aligned rows of a multiple of 256 values");
+  launch_q5(s, w, row_bytes, rows, cols, x, n, y, ys, accumulate);
+  check_launch("gemm_q5_gguf");
+}
 
 bool gemm_kq_supported(int type, int64_t rows, int64_t cols, int n) {
   return (type == kQ4_K || type == kQ6_K) && rows % 32 == 0 && cols % 256 == 0 && n > 8;

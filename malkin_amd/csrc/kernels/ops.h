@@ -55,6 +55,9 @@ bool rows_supported(int type, int64_t cols);
 // The Q4_K / Q5_K panel arithmetic (gemm_avx512.cpp:104-155, 217-266) over GGUF rows: Q5_K's device path.
 void matmul_gguf(hipStream_t s, int type, const void* w, size_t row_bytes, int64_t rows, int64_t cols,
                  const BlockQ8* xq, int n, float* y, int64_t ys, bool accumulate);
+// Q5_K batches over 16-byte aligned GGUF rows on int8 MFMA (gemm_kq.hip); matmul_gguf's choice for more than a few tokens.
+void gemm_q5_gguf(hipStream_t s, const void* w, size_t row_bytes, int64_t rows, int64_t cols, const BlockQ8* x, int n,
+                  float* y, int64_t ys, bool accumulate);
 void matmul_rows(hipStream_t s, int type, const void* w, size_t row_bytes, int64_t rows, int64_t cols, const float* x,
                  int64_t xs, const BlockQ8* xq, int n, float* y, int64_t ys, bool accumulate);
 // gu rows of 2n floats: [gate | up], or (interleave4) gate/up interleaved by 4 as matmul_f32's silu_pairs rows.

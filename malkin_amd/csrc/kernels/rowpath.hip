@@ -8,6 +8,8 @@
 //   bias chains).
 // A wave holds four groups, a workgroup sixteen: one weight row per group, NT tokens of it at once so that a row is read
 // once per token tile. F32 / F16 / BF16 rows go to the matrix cores instead (k_rows_mfma) unless they are unaligned.
+#include <utility>
+
 #include "ctx.h"
 #include "ops.h"
 
@@ -211,7 +213,8 @@ __global__ __launch_bounds__(kRowsThreads) void k_rows(const uint8_t* __restrict
 // read straight from GGUF rows: per output, per 32-value sub-block j in order, acc = fma(float(int dot), (d * sc) * dx,
 // acc), then acc = fma(-(dmin * m), dx * (s0 + s1), acc). An 8-lane group owns one row: lane g takes the 4-value
 // group g of each sub-block, the exact int dot is summed over the group (butterfly), and every lane keeps the same
-// chain. This is the device path for Q5_K weights, which have no CDNA layout.
+// chain. Q5_K weights have no CDNA layout and are read this way; rows that are not 16-byte aligned take this kernel, all
+// others the two below it (k_gguf45_gemv, and gemm_kq.hip's Q5_K form).
 template <bool kHigh>
 __global__ __launch_bounds__(kRowsThreads) void k_gguf45(const uint8_t* __restrict__ W, size_t row_bytes, int64_t rows,
                                                          int64_t cols, const BlockQ8* __restrict__ xq, int n,
@@ -256,6 +259,108 @@ __global__ __launch_bounds__(kRowsThreads) void k_gguf45(const uint8_t* __restri
 #pragma unroll
     for (int t = 0; t < kRowsNT; ++t)
       if (t < nt) {
+        float* o = y + (int64_t)(t0 + t) * ys + r;
+        *o = accumulate ? *o + acc[t] : acc[t];
+      }
+}
+
+// The same arithmetic for up to NT tokens per pass with 16 lanes per row: lane l takes sub-block l % 8 of super-block
+// 2 p + l / 8 whole (16-byte loads, its exact int dot in one lane), so a pass forms the terms of 16 consecutive
+// sub-blocks and the row's chain then runs through them in order, every lane alike, one operand broadcast by the fma's
+// DPP. The next pass's row bytes and activations are loaded while this one runs. What bounds it: the vector work of a
+// pass (about 150 instructions per 4 rows x 512 weights, 1408 bytes) and, with few rows, the chain's 32 dependent
+// fmas. Measured against the byte-wise kernel above (8 lanes per row, the dot summed across lanes per sub-block): Q5_K
+// 2560 x 9728 at one token 200 -> 10 us, 19456 x 2560 71 -> 10.8 (3.2 TB/s); at 4 tokens 371 -> 27 and 126 -> 27.
+template <bool kHigh, int NT>
+__global__ __launch_bounds__(kRowsThreads) void k_gguf45_gemv(const uint8_t* __restrict__ W, size_t row_bytes,
+                                                              int64_t rows, int64_t cols,
+                                                              const BlockQ8* __restrict__ xq, int n,
+                                                              float* __restrict__ y, int64_t ys, int accumulate) {
+  constexpr int kBytes = kHigh ? 176 : 144;
+  const int l = threadIdx.x & 15, j = l & 7;
+  const int64_t r = (int64_t)blockIdx.x * (kRowsThreads / 16) + threadIdx.x / 16;
+  const int t0 = blockIdx.y * NT;
+  const int nsb = (int)(cols / 256), passes = (nsb + 1) / 2;
+  const uint8_t* w = W + (size_t)min(r, rows - 1) * row_bytes;
+  const int64_t nb = cols / 32;
+  struct Pass {
+    uint4 hd, qh[kHigh ? 2 : 1], qs[2];
+    uint2 x[NT][5];
+  };
+  // Never predicated: past the last super-block (or token) the last one again, unused.
+  auto load = [&](Pass& P, int p) __attribute__((always_inline)) {
+    const int sb = min(2 * p + (l >> 3), nsb - 1);
+    const uint8_t* s = w + (size_t)sb * kBytes;
+    P.hd = *reinterpret_cast<const uint4*>(s);
+    if constexpr (kHigh) {
+      P.qh[0] = *reinterpret_cast<const uint4*>(s + 16);
+      P.qh[1] = *reinterpret_cast<const uint4*>(s + 32);
+    }
+    const uint8_t* q = s + (kHigh ? 48 : 16) + 32 * (j >> 1);
+    P.qs[0] = *reinterpret_cast<const uint4*>(q);
+    P.qs[1] = *reinterpret_cast<const uint4*>(q + 16);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const uint2* xb = reinterpret_cast<const uint2*>(xq + (int64_t)min(t0 + t, n - 1) * nb + (int64_t)sb * 8 + j);
+#pragma unroll
+      for (int k = 0; k < 5; ++k) P.x[t][k] = xb[k];
+    }
+  };
+  float acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = 0.0f;
+  auto run = [&](const Pass& P, bool second) __attribute__((always_inline)) {
+    const float d = half_to_float((uint16_t)(P.hd.x & 0xFFFF)), dmin = half_to_float((uint16_t)(P.hd.x >> 16));
+    // scale_min_k4 of sub-block j: the low four take 6 bits of words 1 and 2, the high four nibbles of word 3 and the
+    // top bits of those
+    const int sh = 8 * (j & 3);
+    const uint32_t b1 = P.hd.y >> sh, b2 = P.hd.z >> sh, b3 = P.hd.w >> sh;
+    const uint32_t sc = j < 4 ? b1 & 63u : (b3 & 15u) | ((b1 >> 2) & 0x30u);
+    const uint32_t mn = j < 4 ? b2 & 63u : ((b3 >> 4) & 15u) | ((b2 >> 2) & 0x30u);
+    const float fsc = d * (float)sc, nmn = -(dmin * (float)mn);
+    const uint32_t q[8] = {P.qs[0].x, P.qs[0].y, P.qs[0].z, P.qs[0].w, P.qs[1].x, P.qs[1].y, P.qs[1].z, P.qs[1].w};
+    int v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      v[k] = (int)((q[k] >> (4 * (j & 1))) & 0x0F0F0F0Fu);
+      if constexpr (kHigh) {
+        const uint32_t hb = k < 4 ? (&P.qh[0].x)[k] : (&P.qh[1].x)[k - 4];
+        v[k] |= (int)(((hb >> j) & 0x01010101u) << 4);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      int ai = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        ai = dot4(v[2 * k], (int)P.x[t][k + 1].x, ai);
+        ai = dot4(v[2 * k + 1], (int)P.x[t][k + 1].y, ai);
+      }
+      const float dx = __uint_as_float(P.x[t][0].x);
+      const uint32_t sw = P.x[t][0].y;
+      const float e0 = (float)ai, e1 = fsc * dx, e3 = dx * (float)((int)(int16_t)(sw & 0xFFFF) + (int)(int16_t)(sw >> 16));
+      [&]<int... K>(std::integer_sequence<int, K...>) __attribute__((always_inline)) {
+        ((acc[t] = fma_bcast16<K>(e0, bcast16(e1, K), acc[t]), acc[t] = fma_bcast16<K>(nmn, bcast16(e3, K), acc[t])), ...);
+        if (second)
+          ((acc[t] = fma_bcast16<K + 8>(e0, bcast16(e1, K + 8), acc[t]),
+            acc[t] = fma_bcast16<K + 8>(nmn, bcast16(e3, K + 8), acc[t])),
+           ...);
+      }(std::make_integer_sequence<int, 8>{});
+    }
+  };
+  Pass A, B;
+  load(A, 0);
+  for (int p = 0; p < passes; p += 2) {
+    load(B, min(p + 1, passes - 1));
+    run(A, 2 * p + 1 < nsb);
+    if (p + 1 >= passes) break;
+    load(A, min(p + 2, passes - 1));
+    run(B, 2 * p + 3 < nsb);
+  }
+  if (l == 0 && r < rows)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      if (t0 + t < n) {
         float* o = y + (int64_t)(t0 + t) * ys + r;
         *o = accumulate ? *o + acc[t] : acc[t];
       }
@@ -562,6 +667,30 @@ void matmul_gguf(hipStream_t s, int type, const void* w, size_t row_bytes, int64
           "matmul_gguf: Q4_K / Q5_K rows of a multiple of 256 values");
   require(xq != nullptr, "matmul_gguf: missing activations");
   if (rows <= 0 || n <= 0) return;
+  if (row_bytes % 16 == 0 && (uintptr_t)w % 16 == 0) {
+    // Q5_K batches: the GEMV's waves (4 rows each, a group of 4 tokens) cost about 0.85 us per pass of 512 columns and
+    // wave of a SIMD, the MFMA kernel about 3.1 us per 512 columns whatever the batch (up to 32 tokens), so it takes
+    // over past 3.6 waves per SIMD, i.e. 58 rows x groups per CU. Measured, GEMV / MFMA: 2560 x 9728 at 16 tokens 52 / 60
+    // us, at 24 68 / 68; 19456 x 2560 at 2 tokens 16 / 19, at 4 27 / 19; 5120 x 13824 at 8 70 / 79, at 12 95 / 82;
+    // 1024 x 3072 at 32 15 / 25, at 64 27 / 25; 27648 x 5120 at one token 28 / 35.
+    if (type == kQ5_K && n > 2 && rows * ((n + 3) / 4) > 58 * (int64_t)device_cus()) {
+      gemm_q5_gguf(s, w, row_bytes, rows, cols, xq, n, y, ys, accumulate);
+      return;
+    }
+    auto gemv = [&](auto kern, int nt) {
+      const dim3 grid((unsigned)((rows + kRowsThreads / 16 - 1) / (kRowsThreads / 16)), (unsigned)((n + nt - 1) / nt));
+      hipLaunchKernelGGL(kern, grid, dim3(kRowsThreads), 0, s, static_cast<const uint8_t*>(w), row_bytes, rows, cols,
+                         xq, n, y, ys, accumulate ? 1 : 0);
+    };
+    if (n == 1)
+      type == kQ5_K ? gemv(k_gguf45_gemv<true, 1>, 1) : gemv(k_gguf45_gemv<false, 1>, 1);
+    else if (n == 2)
+      type == kQ5_K ? gemv(k_gguf45_gemv<true, 2>, 2) : gemv(k_gguf45_gemv<false, 2>, 2);
+    else
+      type == kQ5_K ? gemv(k_gguf45_gemv<true, 4>, 4) : gemv(k_gguf45_gemv<false, 4>, 4);
+    check_launch("matmul_gguf");
+    return;
+  }
   const dim3 grid((unsigned)((rows + kRowsThreads / 8 - 1) / (kRowsThreads / 8)), (unsigned)((n + kRowsNT - 1) / kRowsNT));
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(kRowsThreads), 0, s, static_cast<const uint8_t*>(w), row_bytes, rows, cols, xq,
