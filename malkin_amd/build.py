@@ -25,6 +25,7 @@ HIP_SOURCES = [
     "csrc/kernels/gemm_kq.hip",
     "csrc/kernels/quant.hip",
     "csrc/kernels/attn.hip",
+    "csrc/kernels/attn_mma.hip",
     "csrc/kernels/decode.hip",
     "csrc/kernels/cut.hip",
     "csrc/kernels/rowpath.hip",

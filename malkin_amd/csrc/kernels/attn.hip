@@ -831,8 +831,8 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention_grp(const float* __r
   }
 }
 
-// Attention of many query rows at once (prefill and other long plain batches), attend_t semantics for D in {64, 128}
-// and G <= 16, bit-identical to k_attention. A workgroup takes the 16 / G consecutive tokens of one token block and
+// Attention of many query rows at once (prefill and other long plain batches) for the head sizes that attn_mma.hip does
+// not take (D = 64), attend_t semantics, G <= 16, bit-identical to k_attention. A workgroup takes the 16 / G consecutive tokens of one token block and
 // the G query heads of one KV group: up to 16 query rows that share every K and V row they read, so each key is
 // loaded and converted once per 16 rows instead of once per row.
 //   scores  one thread per key: its K row converted to fp32 in registers once, then for each row the 16 lane chains
@@ -1349,7 +1349,17 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
   require(!xq || D % 32 == 0, "attention: Q8 rows need head_dim % 32 == 0");
   const int G = H / KV;
   const bool aligned = attn_aligned(a);
-  if (!anc_off && n >= kRowsMinTokens && G <= 16 && (D == 64 || D == 128) && aligned &&
+  // Many plain tokens on the matrix cores. Rows longer than its LDS holds run their scores twice, which pays where the
+  // grouped kernel (one workgroup per token and KV group) needs more than two rounds of the CUs: 32 heads over 2000 keys
+  // at 32 / 64 / 128 / 256 tokens 47 / 96 / 189 / 380 us grouped, 93 / 98 / 105 / 207 here. (Past the grouped kernel's
+  // keys the caller's scratch must hold a row all the same: such calls have always needed it.)
+  if (!anc_off && n >= kRowsMinTokens && attention_mma_ok(G, D, a) &&
+      (attention_mma_whole(max_keys) ||
+       ((int64_t)n * KV > 2 * device_cus() &&
+        (grp_heads(n, H, G, D, a, anc_off, max_keys) > 0 ||
+         (scratch && scratch_bytes >= 2 * (size_t)attn_keys_pad(max_keys) * sizeof(float)))))) {
+    attention_mma(s, q, q_stride, out, out_stride, n, G, KV, scale, a, seq, n_keys, max_keys, xq, xq_stride);
+  } else if (!anc_off && n >= kRowsMinTokens && G <= 16 && D == 64 && a.k_perm && aligned &&
       rows_lds_bytes(D, attn_keys_pad(max_keys)) <= 160 * 1024 - 1024) {
     const int nk_pad = attn_keys_pad(max_keys);
     const size_t lds = rows_lds_bytes(D, nk_pad);
@@ -1365,10 +1375,7 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
       hipLaunchKernelGGL(kernel, dim3(((n + TQ - 1) / TQ) * KV), dim3(kRowsThreads), lds, s, q, q_stride, out,
                          out_stride, G, scale, a, seq, n_keys, n, KV, nk_pad, xq, xq_stride);
     };
-    if (D == 64)
-      a.k_perm ? go(k_attention_rows<64, true>) : go(k_attention_rows<64, false>);
-    else
-      a.k_perm ? go(k_attention_rows<128, true>) : go(k_attention_rows<128, false>);
+    go(k_attention_rows<64, true>);
   } else if (!anc_off && dec_ok(G, D, a, max_keys)) {
     launch_dec<false>(s, q, q_stride, out, out_stride, n, H, D, G, scale, a, seq, n_keys, max_keys, DecFuse{}, xq,
                       xq_stride);

@@ -132,6 +132,13 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
                const AttnAddr& a, const int32_t* seq, const int32_t* n_keys, const int32_t* anc_off,
                const int32_t* anc, int max_keys, void* scratch, size_t scratch_bytes, BlockQ8* xq = nullptr,
                int64_t xq_stride = 0);
+// Plain batches of many tokens at head_dim 128 over the permuted device cache (attn_mma.hip); attention()'s choice from
+// 16 tokens on.
+bool attention_mma_ok(int G, int D, const AttnAddr& a);
+bool attention_mma_whole(int max_keys);  // a row's scores fit LDS (else they are computed twice)
+void attention_mma(hipStream_t s, const float* q, int64_t q_stride, float* out, int64_t out_stride, int n, int G, int KV,
+                   float scale, const AttnAddr& a, const int32_t* seq, const int32_t* n_keys, int max_keys, BlockQ8* xq,
+                   int64_t xq_stride);
 // Scratch the attention of `pairs` (token, head) pairs over max_keys keys uses (0: none).
 size_t attention_scratch_bytes(int D, int max_keys, int pairs);
 
