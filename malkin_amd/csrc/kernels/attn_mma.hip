@@ -244,7 +244,7 @@ __global__ __launch_bounds__(kThreads) void k_attention_mma(const float* __restr
       put_max();
     }
     const int sr = tid >> 5, sx = tid & 31;  // softmax: threads 32 r .. 32 r + 31 of row r
-    const int nkr = sr < R && ((act >> sr) & 1) ? nk_s[sr] : 0;
+    const int nkr = sr < R && ((act >> sr) & 1) ? min(nk_s[sr], nkb) : 0;
     float lane_sum = 0.0f;  // threads x < 16 of a row: lane x's sequential sum
     v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};  // P.V: values 16 w + li of rows 4 lq + i
     for (int k0 = 0; k0 < nkb; k0 += nk_pad) {
@@ -256,17 +256,18 @@ __global__ __launch_bounds__(kThreads) void k_attention_mma(const float* __restr
       for (int c = st0; c < st0 + kVStages - 1 && c < st1; ++c) v_issue(c);  // in flight during the softmax
 
       // softmax_inplace (kernels_avx512.cpp:205-226): two keys, 16 apart, on lanes x and x + 16 per 32 keys, added in
-      // that order by lane x. Past the row's end e = +0, which leaves the sum unchanged.
+      // that order by lane x. Past the row's end e = +0, which leaves the sum unchanged, and so is the coefficient,
+      // whatever the scales of keys that only other rows have (0 * inf).
       {
         float m = max_s[0][sr];
 #pragma unroll
         for (int i = 1; i < kWaves; ++i) m = fmaxf(m, max_s[i][sr]);
         float* srow = sc + sr * S;
-        const int real = 16 * tl - k0;  // keys with a v scale
         auto one = [&](int j) __attribute__((always_inline)) {
           const int at = key_pos(j);
-          const float e = k0 + j < nkr ? exp512(srow[at] - m) : 0.0f;
-          srow[at] = e * (j < real ? vsc[at] : 0.0f);
+          const bool in = k0 + j < nkr;
+          const float e = in ? exp512(srow[at] - m) : 0.0f;
+          srow[at] = in ? e * vsc[at] : 0.0f;
           return e;
         };
         for (int j = sx; j < held; j += 64) {
@@ -371,21 +372,21 @@ void attention_mma(hipStream_t s, const float* q, int64_t q_stride, float* out, 
                    float scale, const AttnAddr& a, const int32_t* seq, const int32_t* n_keys, int max_keys, BlockQ8* xq,
                    int64_t xq_stride) {
   const int TQ = kRows / G, max_pad = pad64(max_keys);
-  auto go = [&](auto kernel, int nk_pad) {
+  auto go = [&]<bool LONG>(int nk_pad) {
     static bool attr = false;  // per instantiation
     if (!attr) {
-      check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)kLds),
+      check(hipFuncSetAttribute(reinterpret_cast<const void*>(k_attention_mma<LONG>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds),
             "hipFuncSetAttribute");
       attr = true;
     }
-    hipLaunchKernelGGL(kernel, dim3(((n + TQ - 1) / TQ) * KV), dim3(kThreads), mma_lds_bytes(nk_pad), s, q, q_stride,
+    hipLaunchKernelGGL(k_attention_mma<LONG>, dim3(((n + TQ - 1) / TQ) * KV), dim3(kThreads), mma_lds_bytes(nk_pad), s, q, q_stride,
                        out, out_stride, G, scale, a, seq, n_keys, n, KV, max_pad, xq, xq_stride);
   };
   if (attention_mma_whole(max_keys))
-    go(k_attention_mma<false>, max_pad);
+    go.template operator()<false>(max_pad);
   else
-    go(k_attention_mma<true>, kChunk);
+    go.template operator()<true>(kChunk);
   check_launch("attention_mma");
 }
 
