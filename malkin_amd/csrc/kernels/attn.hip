@@ -831,10 +831,11 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention_grp(const float* __r
   }
 }
 
-// Attention of many query rows at once (prefill and other long plain batches) for the head sizes that attn_mma.hip does
-// not take (D = 64), attend_t semantics, G <= 16, bit-identical to k_attention. A workgroup takes the 16 / G consecutive tokens of one token block and
-// the G query heads of one KV group: up to 16 query rows that share every K and V row they read, so each key is
-// loaded and converted once per 16 rows instead of once per row.
+// Attention of many query rows at once (prefill and other long plain batches) for the head size that attn_mma.hip does
+// not take (D = 64), attend_t semantics, G <= 16, over the permuted device cache, bit-identical to k_attention. A
+// workgroup takes the 16 / G consecutive tokens of one token block and the G query heads of one KV group: up to 16 query
+// rows that share every K and V row they read, so each key is loaded and converted once per 16 rows instead of once per
+// row.
 //   scores  one thread per key: its K row converted to fp32 in registers once, then for each row the 16 lane chains
 //           (mul, then fma over the D/16 chunks), the halving tree, times (kv_scale * scale). q is uniform over the
 //           workgroup and is read through the scalar unit;
@@ -865,7 +866,7 @@ __host__ __device__ constexpr size_t rows_lds_bytes(int D, int nk_pad) {
   return 4 * (2 * (size_t)(4096 / D) * (size_t)(D + 4) + (size_t)(kRowsMax + 1) * (size_t)nk_pad);
 }
 
-template <int D, bool PERM>
+template <int D>
 __global__ __launch_bounds__(kRowsThreads) void k_attention_rows(const float* __restrict__ q, int64_t q_stride,
                                                                  float* __restrict__ out, int64_t out_stride, int G,
                                                                  float scale, AttnAddr a,
@@ -942,7 +943,7 @@ __global__ __launch_bounds__(kRowsThreads) void k_attention_rows(const float* __
       for (int l = 0; l < 16; ++l)
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
-          const int e = PERM ? DC * l + c : 16 * c + l;  // byte of element 16 c + l
+          const int e = DC * l + c;  // byte of element 16 c + l
           kf[l][c] = (float)(int8_t)(kw[e >> 4][(e >> 2) & 3] >> (8 * (e & 3)));
         }
       if (live) vsc[j] = vsv;
@@ -1360,22 +1361,17 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
          (scratch && scratch_bytes >= 2 * (size_t)attn_keys_pad(max_keys) * sizeof(float)))))) {
     attention_mma(s, q, q_stride, out, out_stride, n, G, KV, scale, a, seq, n_keys, max_keys, xq, xq_stride);
   } else if (!anc_off && n >= kRowsMinTokens && G <= 16 && D == 64 && a.k_perm && aligned &&
-      rows_lds_bytes(D, attn_keys_pad(max_keys)) <= 160 * 1024 - 1024) {
-    const int nk_pad = attn_keys_pad(max_keys);
-    const size_t lds = rows_lds_bytes(D, nk_pad);
-    auto go = [&](auto kernel) {
-      static bool attr = false;
-      if (!attr) {
-        check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  160 * 1024 - 1024),
-              "hipFuncSetAttribute");
-        attr = true;
-      }
-      const int TQ = kRowsMax / G;
-      hipLaunchKernelGGL(kernel, dim3(((n + TQ - 1) / TQ) * KV), dim3(kRowsThreads), lds, s, q, q_stride, out,
-                         out_stride, G, scale, a, seq, n_keys, n, KV, nk_pad, xq, xq_stride);
-    };
-    go(k_attention_rows<64, true>);
+             rows_lds_bytes(D, attn_keys_pad(max_keys)) <= 160 * 1024 - 1024) {
+    const int nk_pad = attn_keys_pad(max_keys), TQ = kRowsMax / G;
+    static bool attr = false;
+    if (!attr) {
+      check(hipFuncSetAttribute(reinterpret_cast<const void*>(k_attention_rows<64>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 1024),
+            "hipFuncSetAttribute");
+      attr = true;
+    }
+    hipLaunchKernelGGL(k_attention_rows<64>, dim3(((n + TQ - 1) / TQ) * KV), dim3(kRowsThreads), rows_lds_bytes(D, nk_pad),
+                       s, q, q_stride, out, out_stride, G, scale, a, seq, n_keys, n, KV, nk_pad, xq, xq_stride);
   } else if (!anc_off && dec_ok(G, D, a, max_keys)) {
     launch_dec<false>(s, q, q_stride, out, out_stride, n, H, D, G, scale, a, seq, n_keys, max_keys, DecFuse{}, xq,
                       xq_stride);
