@@ -23,7 +23,6 @@ namespace {
 
 constexpr int kSelThreads = 1024;            // k_topk_final
 constexpr int kPartThreads = 256;            // k_topk_part
-constexpr int kPartPer = 16;                 // logits per thread and round of k_topk_part
 constexpr int kFinalPer = 8;                 // keys per thread (and round) of k_topk_final
 constexpr int kMaxTopK = 1024;               // candidates per row held in LDS
 constexpr int kSlices = 64, kChunk = 64;     // slice p of a row: its chunks p, p + kSlices, ...
@@ -32,6 +31,11 @@ constexpr int kOneSlice = kFinalPer * kSelThreads;  // logits of a row that one 
 // Candidates that a slice gives: four times the k / kSlices it holds on average, and 16.
 __host__ __device__ constexpr int slice_keep(int k) { return k < 16 + k / 16 ? k : 16 + k / 16; }
 static_assert(kSlices * slice_keep(kMaxTopK) <= kFinalPer * kSelThreads, "one workgroup holds a row's candidates");
+
+// Logits of a slice, some of them past the row's end.
+__host__ __device__ constexpr int slice_logits(int n_vocab) {
+  return (int)((n_vocab + (int64_t)kSlices * kChunk - 1) / (kSlices * kChunk)) * kChunk;
+}
 
 // Larger float -> larger key, never 0 (finite values and infinities; NaN logits are not expected).
 __device__ __forceinline__ uint32_t order_key(float f) {
@@ -51,12 +55,14 @@ __global__ void k_penalize(float* __restrict__ logits, int64_t stride, const int
   }
 }
 
-// The k-th largest of the workgroup's keys (E per thread), i.e. the largest T with at least k keys >= T: two bits per
-// step from the top, the counts of the three candidate values by wave ballots and one LDS add per wave. cnt: kSteps
-// groups of 3 zeroed counters, fresh ones per step, so that one barrier per step suffices. k >= 1; keys >= k.
+// A T that separates the k largest of the workgroup's keys (E per thread): the largest T with at least k keys >= T, or
+// any with exactly k. Two bits per step from the top, the counts of the three candidate values by wave ballots and one
+// LDS add per wave; the search ends at the first prefix that k keys reach exactly (without ties about half of the 16
+// steps: 8 rows of 151936 random logits at k = 40 29.5 -> 23.2 us). cnt: kSteps groups of 3 zeroed counters, fresh ones per
+// step, so that one barrier per step suffices. k >= 1; where fewer keys are not 0, T = 0.
 constexpr int kSteps = 16;
 template <int E>
-__device__ __forceinline__ uint32_t kth_largest(const uint32_t (&key)[E], uint32_t k, uint32_t* cnt) {
+__device__ __forceinline__ uint32_t separate(const uint32_t (&key)[E], uint32_t k, uint32_t* cnt) {
   uint32_t T = 0;
   for (int st = 0; st < kSteps; ++st) {
     const int shift = 30 - 2 * st;
@@ -73,6 +79,7 @@ __device__ __forceinline__ uint32_t kth_largest(const uint32_t (&key)[E], uint32
     const uint32_t *g = cnt + 3 * st;
     const uint32_t v = g[2] >= k ? 3u : g[1] >= k ? 2u : g[0] >= k ? 1u : 0u;
     T |= v << shift;
+    if (v != 0 && g[v - 1] == k) break;
   }
   return T;
 }
@@ -92,7 +99,7 @@ __device__ __forceinline__ int select_k(const uint32_t (&key)[E], const int32_t 
   if (tid < 2 * 3 * kSteps) (&L.cnt[0][0])[tid] = 0;
   if (tid == 0) L.gt = L.eq = L.slot = 0;
   __syncthreads();
-  const uint32_t T = kth_largest(key, (uint32_t)k, L.cnt[0]);
+  const uint32_t T = separate(key, (uint32_t)k, L.cnt[0]);
   uint32_t ngt = 0, neq = 0;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
@@ -104,14 +111,15 @@ __device__ __forceinline__ int select_k(const uint32_t (&key)[E], const int32_t 
     if (neq) atomicAdd(&L.eq, neq);
   }
   __syncthreads();
-  // Of the keys equal to T, the need lowest ids: those with ~id at least the need-th largest ~id among them.
+  // Of the keys equal to T, the need lowest ids: those with the need largest ~id among them (all of them where T
+  // already separates k keys).
   const uint32_t need = (uint32_t)k - L.gt;
   uint32_t U = 0;
   if (T != 0 && L.eq > need) {
     uint32_t inv[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) inv[e] = key[e] == T ? ~(uint32_t)id[e] : 0u;
-    U = kth_largest(inv, need, L.cnt[1]);
+    U = separate(inv, need, L.cnt[1]);
   }
 #pragma unroll
   for (int e = 0; e < E; ++e) {
@@ -128,16 +136,17 @@ __device__ __forceinline__ int select_k(const uint32_t (&key)[E], const int32_t 
 
 // Slice p of a row: its slice_keep(k) first candidates (all of them, then (0, INT32_MAX), where it holds no more) to
 // cand[row][p][keep]. A slice of more logits than the threads hold is walked in rounds, each over the candidates so far
-// and the next logits.
+// and the next logits. E: logits per thread and round.
+template <int E>
 __global__ __launch_bounds__(kPartThreads) void k_topk_part(const float* __restrict__ logits, int64_t stride,
                                                              const int32_t* __restrict__ rows, int n_vocab, int keep,
                                                              uint2* cand) {
-  constexpr int E = kPartPer, NT = kPartThreads;
+  constexpr int NT = kPartThreads;
   __shared__ SelLds L;
   const int tid = threadIdx.x, r = blockIdx.y, p = blockIdx.x;
   const float* l = logits + (int64_t)(rows ? rows[r] : r) * stride;
   auto at = [&](int j) { return ((int64_t)(j / kChunk) * kSlices + p) * kChunk + j % kChunk; };  // slice logit j
-  const int n = (int)((n_vocab + (int64_t)kSlices * kChunk - 1) / (kSlices * kChunk)) * kChunk;  // some past n_vocab
+  const int n = slice_logits(n_vocab);
   uint2* out = cand + ((int64_t)r * kSlices + p) * keep;
   uint32_t key[E];
   int32_t id[E];
@@ -289,9 +298,10 @@ void penalize(hipStream_t s, float* logits, int64_t stride, const int32_t* rows,
 
 // Rows of up to kOneSlice logits take one workgroup each; longer ones kSlices slices, whose candidates go through the
 // scratch, as many rows per pair of launches as it holds (40 KB per row at k = 1024). Measured, with one
-// workgroup walking each row -> this form: 8 rows of 151936 at k = 40 267 -> 29.5 us (1024: 276 -> 55), one row
-// 203 -> 25, 64 rows 384 -> 115, 8 rows of 8193 60 -> 28; of 8192, which one workgroup selects from registers in one
-// round (slices would cost the second launch), 57 -> 17.
+// workgroup walking each row -> this form: 8 rows of 151936 at k = 40 276 -> 23 us (1024: 287 -> 48), one row
+// 238 -> 18, 64 rows 407 -> 72, 8 rows of 8193 56 -> 14; of 8192, which one workgroup selects from registers in one
+// round (slices would cost the second launch), 57 -> 17 before the searches ended early. A slice's threads hold 4, 8, 12
+// or 16 logits each, as many as it needs: the searches' ballots are what k_topk_part spends its time on.
 void topk(hipStream_t s, const float* logits, int64_t stride, const int32_t* rows, int n_rows, int n_vocab, int k,
           float* out_v, int32_t* out_i, void* scratch, size_t scratch_bytes) {
   if (n_rows <= 0) return;
@@ -305,8 +315,16 @@ void topk(hipStream_t s, const float* logits, int64_t stride, const int32_t* row
     const int nr = std::min(batch, n_rows - r0);
     const float* l = rows ? logits : logits + (int64_t)r0 * stride;
     const int32_t* rr = rows ? rows + r0 : nullptr;
-    if (sliced)
-      hipLaunchKernelGGL(k_topk_part, dim3(kSlices, nr), dim3(kPartThreads), 0, s, l, stride, rr, n_vocab, keep, cand);
+    auto part = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(kSlices, nr), dim3(kPartThreads), 0, s, l, stride, rr, n_vocab, keep, cand);
+    };
+    if (sliced) {
+      const int per = (slice_logits(n_vocab) + kPartThreads - 1) / kPartThreads;
+      per <= 4    ? part(k_topk_part<4>)
+      : per <= 8  ? part(k_topk_part<8>)
+      : per <= 12 ? part(k_topk_part<12>)
+                  : part(k_topk_part<16>);
+    }
     hipLaunchKernelGGL(k_topk_final, dim3(nr), dim3(kSelThreads), 0, s, l, stride, rr, n_vocab, cand, k,
                        out_v + (int64_t)r0 * k, out_i + (int64_t)r0 * k);
   }

@@ -1,6 +1,8 @@
 """mk_topk where its forms meet: rows that one workgroup takes alone (up to 8192 logits), rows cut into 64 slices, slices
-walked in rounds (more than 4096 logits each), rows whose largest logits fall into one slice (the row is then walked
-whole), and more rows than the context's scratch holds candidates for, against numpy's stable order."""
+of 4, 8, 12 or 16
+logits a thread, slices walked in rounds (more than 4096 logits each), rows whose largest logits fall into one slice
+(the row is then walked whole), and more rows than the context's scratch holds candidates for, against numpy's stable
+order."""
 import numpy as np
 import pytest
 
@@ -11,6 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("V,k,n_rows", [(8192, 1024, 2), (8193, 257, 2), (8193, 1024, 5), (32 * 1024 + 5, 1, 2),
+                                        (65536, 40, 3), (65537, 700, 3), (131072, 40, 3), (131073, 999, 3),
+                                        (196608, 40, 3), (196609, 500, 3),
                                         (64 * 4096, 300, 3), (64 * 4096 + 1, 300, 3), (64 * 4096 + 64, 1024, 3),
                                         (1 << 20, 1000, 3), (20000, 128, 70), (20000, 129, 3), (151936, 1024, 30)])
 def test_topk_forms(mk, V, k, n_rows):
