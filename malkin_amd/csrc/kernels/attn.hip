@@ -96,6 +96,79 @@ __global__ __launch_bounds__(64) void k_qk_norm_rope_kv(float* __restrict__ q, f
   if (lane == 0) (is_v ? kv.vs : kv.ks)[row] = d;
 }
 
+// The same for D = 128 with 16 lanes per (token, head) and no LDS: lane l holds the elements 16 c + l, c = 0..7, which are
+// chain l of the norm's sum of squares, both halves of its four RoPE pairs (c and c + 4), and the eight bytes 8 l .. of
+// a permuted K row. A value head has neither, so its lanes take eight consecutive elements. One 64-thread workgroup and
+// five barriers per head bound the kernel above; this one, for prompts, the bytes it moves: 512 tokens of 48 heads
+// (25 MB) 11.0 -> 6.2 us; for a few tokens both take a launch.
+constexpr int kQk128Threads = 256;
+__global__ __launch_bounds__(kQk128Threads) void k_qk_norm_rope_kv128(
+    float* __restrict__ q, float* __restrict__ k, const float* __restrict__ v, int64_t stride, int n, int H, int KV,
+    const float* __restrict__ q_norm, const float* __restrict__ k_norm, float eps, const float* __restrict__ cos_t,
+    const float* __restrict__ sin_t, const int32_t* __restrict__ rpos, const int32_t* __restrict__ seq,
+    const int32_t* __restrict__ kv_row, KvLayer kv, int n_ctx) {
+  constexpr int D = 128;
+  const int l = threadIdx.x & 15, nh = H + 2 * KV;
+  const int64_t it = (int64_t)blockIdx.x * (kQk128Threads / 16) + threadIdx.x / 16;
+  if (it >= (int64_t)n * nh) return;  // whole 16-lane groups leave
+  const int t = (int)(it / nh), hh = (int)(it % nh);
+  const bool is_q = hh < H, is_v = hh >= H + KV;
+  const int head = is_q ? hh : is_v ? hh - H - KV : hh - H;
+  float x[8];
+  if (is_v) {
+    const float* src = v + t * stride + (int64_t)head * D + 8 * l;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const float4 f = *reinterpret_cast<const float4*>(src + 4 * c);
+      x[4 * c] = f.x, x[4 * c + 1] = f.y, x[4 * c + 2] = f.z, x[4 * c + 3] = f.w;
+    }
+  } else {
+    float* vec = (is_q ? q : k) + t * stride + (int64_t)head * D + l;
+    const float* w = (is_q ? q_norm : k_norm) + l;
+    const int64_t pos = rpos[t];
+    float wv[8], cv[4], sv[4];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) x[c] = vec[16 * c];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) wv[c] = w[16 * c];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      cv[c] = cos_t[pos * (D / 2) + 16 * c + l];
+      sv[c] = sin_t[pos * (D / 2) + 16 * c + l];
+    }
+    float acc = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) acc = fma_(x[c], x[c], acc);
+    acc = __shfl(reduce16_lanes(acc), 0, 16);
+    const float s = 1.0f / sqrtf(acc / (float)D + eps);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) x[c] = x[c] * s * wv[c];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float x0 = x[c], x1 = x[c + 4];
+      x[c] = fma_(x0, cv[c], -(x1 * sv[c]));
+      x[c + 4] = fma_(x0, sv[c], x1 * cv[c]);
+    }
+    if (is_q) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) vec[16 * c] = x[c];
+      return;
+    }
+  }
+  float amax = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) amax = fmaxf(amax, fabsf(x[c]));
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 16));
+  const float d = amax / 127.0f, id = d != 0.0f ? 1.0f / d : 0.0f;
+  const int64_t row = ((int64_t)seq[t] * KV + head) * n_ctx + kv_row[t];
+  uint32_t b[2] = {0, 0};
+#pragma unroll
+  for (int c = 0; c < 8; ++c) b[c >> 2] |= (uint32_t)(uint8_t)(int8_t)(int)__builtin_rintf(x[c] * id) << (8 * (c & 3));
+  *reinterpret_cast<uint2*>((is_v ? kv.v : kv.k) + row * D + 8 * l) = make_uint2(b[0], b[1]);
+  if (l == 0) (is_v ? kv.vs : kv.ks)[row] = d;
+}
+
 // Attention of one query head per workgroup, attend_t semantics (D in {64,128,256}, G <= 16):
 //   scores  the 16 lane chains of attend_t (mul, then fma over D/16 chunks), the halving tree, times
 //           (kv_scale * scale). Permuted K rows (the device cache): 16 lanes per key, lane l holding the D/16 values
@@ -1264,6 +1337,14 @@ void qk_norm_rope_kv(hipStream_t s, float* q, float* k, const float* v, int64_t 
                      const int32_t* rpos, const int32_t* seq, const int32_t* kv_row, const KvLayer& kv, int n_ctx) {
   if (n <= 0) return;
   require(D % 16 == 0 && D <= 64 * kQkMaxPer, "qk_norm_rope_kv: head_dim must be a multiple of 16, at most 256");
+  const auto aligned = [](const void* p, int b) { return reinterpret_cast<uintptr_t>(p) % b == 0; };
+  const int64_t groups = ((int64_t)n * (H + 2 * KV) + kQk128Threads / 16 - 1) / (kQk128Threads / 16);
+  if (D == 128 && aligned(v, 16) && stride % 4 == 0 && aligned(kv.k, 8) && aligned(kv.v, 8) && groups < INT32_MAX) {
+    hipLaunchKernelGGL(k_qk_norm_rope_kv128, dim3((unsigned)groups), dim3(kQk128Threads), 0, s, q, k, v, stride, n, H, KV,
+                       q_norm, k_norm, eps, cos_t, sin_t, rpos, seq, kv_row, kv, n_ctx);
+    check_launch("qk_norm_rope_kv");
+    return;
+  }
   hipLaunchKernelGGL(k_qk_norm_rope_kv, dim3(n, H + 2 * KV), dim3(64), D * sizeof(float), s, q, k, v, stride, H, KV,
                      D, q_norm, k_norm, eps, cos_t, sin_t, rpos, seq, kv_row, kv, n_ctx);
   check_launch("qk_norm_rope_kv");
