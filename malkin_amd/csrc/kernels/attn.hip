@@ -556,9 +556,10 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention_long(const float* __
   }
 }
 
-// GH query heads of one KV group for one token per workgroup (GH = G = 2..5, or GH = 1; D = 128, permuted K rows,
-// the keys in LDS): verification trees and contexts past the decode kernel's LDS. With GH = G every K and V row is
-// read, converted and staged once for the G heads instead of G times. Same arithmetic as attend_pair, head by head:
+// GH query heads of one KV group for one token per workgroup (GH = 1..G, at most 5; D = 128, permuted K rows, the keys
+// in LDS): verification trees and contexts past the decode kernel's LDS. Every K and V row is read, converted and staged
+// once for the GH heads instead of GH times. Where GH does not divide G the last workgroup's heads reach back into the
+// one's before it, and only that one stores those. Same arithmetic as attend_pair, head by head:
 //   scores  16 lanes per key as in attend_pair; each lane holds the D/16 q values of its chain for every head and
 //           runs G dot products on the K bytes it loaded once;
 //   softmax per head, one pass over the keys for all heads (G maxima, one barrier);
@@ -602,7 +603,7 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention_grp(const float* __r
   const int tid = threadIdx.x;
   // (group, token, head subset) numbered group-major; XCD x (workgroups x, x + 8, ...) takes a contiguous run, so a
   // group's K/V rows are read into one XCD's L2.
-  const int hs = G / GH;  // head subsets per group
+  const int hs = (G + GH - 1) / GH;  // head subsets per group
   int t, g, hsub;
   {
     const int total = n * KV * hs, w = (int)blockIdx.x;
@@ -611,7 +612,8 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention_grp(const float* __r
     t = (pair / hs) % n;
     hsub = pair % hs;
   }
-  const int hfirst = g * G + hsub * GH;  // the workgroup's first query head
+  const int hfirst = g * G + min(hsub * GH, G - GH);  // the workgroup's first query head
+  const int hout = g * G + hsub * GH;                 // the first one it stores
   const int n0 = n_keys[t];
   const int e0 = anc_off ? anc_off[t] : 0, ne = anc_off ? anc_off[t + 1] - e0 : 0;
   const int nk = n0 + ne;
@@ -900,7 +902,7 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention_grp(const float* __r
     float* o = out + t * out_stride + (int64_t)(hfirst + hb) * D + d;
 #pragma unroll
     for (int k = 0; k < C::h0; ++k)
-      if (k < nh) put_out(o + k * D - d, xq, t * xq_stride, (hfirst + hb + k) * D, d, acc[k] * inv_s[hb + k]);
+      if (k < nh && hfirst + hb + k >= hout) put_out(o + k * D - d, xq, t * xq_stride, (hfirst + hb + k) * D, d, acc[k] * inv_s[hb + k]);
   }
 }
 
@@ -1410,15 +1412,20 @@ size_t attention_scratch_bytes(int D, int max_keys, int pairs) {
   return (size_t)std::min(pairs, 1024) * 2 * (size_t)nk_pad * sizeof(float);
 }
 
-// Heads per workgroup of the grouped kernel for this batch (0: not used). All G heads of a KV group (G = 2..5) when one
-// workgroup per (token, head) would take more than one round of the CUs: a grouped workgroup costs about twice a
-// single-head one (2057 keys, G = 5: 62 vs 31 us), so with fewer pairs than CUs one head per workgroup is faster.
+// Heads per workgroup of the grouped kernel for this batch (0: not used): the fewest with which the workgroups take one
+// round of the CUs (each holds a CU: 1024 threads), else all G heads (G <= 5); a second round would cost more than fewer
+// heads save (2057 keys: 31 us for one head, 62 for five). The attention half of a layer over 2048 keys, all heads -> this
+// split: 5 heads a group, 7 tokens (2 heads a workgroup) 97 -> 80 us, 13 (3) 110 -> 100; 4 heads, 9 and 15 tokens (2)
+// 87 -> 78 and 88 -> 80.
 int grp_heads(int n, int H, int G, int D, const AttnAddr& a, const int32_t* anc_off, int max_keys) {
   if (D != 128 || !a.k_perm || !attn_aligned(a) || G > 16) return 0;
   const int nk_pad = attn_keys_pad(max_keys), anc_cap = anc_off ? std::min(n, nk_pad) : 0;
   const size_t limit = 160 * 1024 - 1024;
-  if (G >= 2 && G <= kGrpMaxHeads && (int64_t)n * H > device_cus() && grp_lds_bytes(G, nk_pad, anc_cap) <= limit)
-    return G;
+  if (G <= kGrpMaxHeads) {
+    int GH = 1;
+    while (GH < G && (int64_t)n * (H / G) * ((G + GH - 1) / GH) > device_cus()) ++GH;
+    if (grp_lds_bytes(GH, nk_pad, anc_cap) <= limit) return GH;
+  }
   return grp_lds_bytes(1, nk_pad, anc_cap) <= limit ? 1 : 0;
 }
 
@@ -1457,8 +1464,7 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
     launch_dec<false>(s, q, q_stride, out, out_stride, n, H, D, G, scale, a, seq, n_keys, max_keys, DecFuse{}, xq,
                       xq_stride);
   } else if (grp_heads(n, H, G, D, a, anc_off, max_keys) > 0) {
-    // Grouped workgroups (trees, keys past the decode kernel's LDS): all heads of a KV group per workgroup where one
-    // workgroup per (token, head) would take more than one round of the CUs, else one head per workgroup.
+    // Grouped workgroups (trees, keys past the decode kernel's LDS).
     const int GH = grp_heads(n, H, G, D, a, anc_off, max_keys);
     const int nk_pad = attn_keys_pad(max_keys), anc_cap = anc_off ? std::min(n, nk_pad) : 0;
     const size_t lds = grp_lds_bytes(GH, nk_pad, anc_cap);
@@ -1470,7 +1476,7 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
               "hipFuncSetAttribute");
         done = true;
       }
-      hipLaunchKernelGGL(kernel, dim3(n * KV * (G / GH)), dim3(kAttnThreads), lds, s, q, q_stride, out, out_stride, G,
+      hipLaunchKernelGGL(kernel, dim3(n * KV * ((G + GH - 1) / GH)), dim3(kAttnThreads), lds, s, q, q_stride, out, out_stride, G,
                          scale, a, seq, n_keys, anc_off, anc, n, KV, nk_pad, anc_cap, xq, xq_stride);
     };
     switch (GH) {
