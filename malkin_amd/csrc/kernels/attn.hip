@@ -1354,6 +1354,8 @@ void qk_norm_rope_kv(hipStream_t s, float* q, float* k, const float* v, int64_t 
 
 namespace {
 
+constexpr int kLdsLimit = 160 * 1024 - 1024;  // dynamic LDS of a launch
+
 bool dec_ok(int G, int D, const AttnAddr& a, int max_keys) {
   return G <= 16 && (D == 64 || D == 128) && a.k_perm && attn_aligned(a) && dec_fits(D, max_keys);
 }
@@ -1363,26 +1365,20 @@ void launch_dec(hipStream_t s, const float* q, int64_t q_stride, float* out, int
                 int G, float scale, const AttnAddr& a, const int32_t* seq, const int32_t* n_keys, int max_keys,
                 const DecFuse& f, BlockQ8* xq, int64_t xq_stride) {
   const size_t lds = dec_lds_bytes(D, attn_keys_pad(max_keys));
-  auto go = [&](auto kernel) {
-    static bool attr = false;
-    if (!attr) {
-      check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                160 * 1024 - 1024),
-            "hipFuncSetAttribute");
-      attr = true;
-    }
-    hipLaunchKernelGGL(kernel, dim3(n * H), dim3(kDecThreads), lds, s, q, q_stride, out, out_stride, G, scale, a, seq,
-                       n_keys, n, H, f, xq, xq_stride);
+  auto go = [&]<int DD, int SLOTS>() {
+    allow_lds<k_attention_dec<DD, SLOTS, FUSE>>(kLdsLimit);
+    hipLaunchKernelGGL((k_attention_dec<DD, SLOTS, FUSE>), dim3(n * H), dim3(kDecThreads), lds, s, q, q_stride, out,
+                       out_stride, G, scale, a, seq, n_keys, n, H, f, xq, xq_stride);
   };
   const int slots = dec_slots(D, max_keys, FUSE);
   if (D == 64) {
-    slots == 1   ? go(k_attention_dec<64, 1, FUSE>)
-    : slots == 2 ? go(k_attention_dec<64, 2, FUSE>)
-                 : go(k_attention_dec<64, 3, FUSE>);
+    slots == 1   ? go.template operator()<64, 1>()
+    : slots == 2 ? go.template operator()<64, 2>()
+                 : go.template operator()<64, 3>();
   } else {
-    slots == 1   ? go(k_attention_dec<128, 1, FUSE>)
-    : slots == 2 ? go(k_attention_dec<128, 2, FUSE>)
-                 : go(k_attention_dec<128, 3, FUSE>);
+    slots == 1   ? go.template operator()<128, 1>()
+    : slots == 2 ? go.template operator()<128, 2>()
+                 : go.template operator()<128, 3>();
   }
 }
 
@@ -1451,13 +1447,7 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
   } else if (!anc_off && n >= kRowsMinTokens && G <= 16 && D == 64 && a.k_perm && aligned &&
              rows_lds_bytes(D, attn_keys_pad(max_keys)) <= 160 * 1024 - 1024) {
     const int nk_pad = attn_keys_pad(max_keys), TQ = kRowsMax / G;
-    static bool attr = false;
-    if (!attr) {
-      check(hipFuncSetAttribute(reinterpret_cast<const void*>(k_attention_rows<64>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 1024),
-            "hipFuncSetAttribute");
-      attr = true;
-    }
+    allow_lds<k_attention_rows<64>>(kLdsLimit);
     hipLaunchKernelGGL(k_attention_rows<64>, dim3(((n + TQ - 1) / TQ) * KV), dim3(kRowsThreads), rows_lds_bytes(D, nk_pad),
                        s, q, q_stride, out, out_stride, G, scale, a, seq, n_keys, n, KV, nk_pad, xq, xq_stride);
   } else if (!anc_off && dec_ok(G, D, a, max_keys)) {
@@ -1468,49 +1458,37 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
     const int GH = grp_heads(n, H, G, D, a, anc_off, max_keys);
     const int nk_pad = attn_keys_pad(max_keys), anc_cap = anc_off ? std::min(n, nk_pad) : 0;
     const size_t lds = grp_lds_bytes(GH, nk_pad, anc_cap);
-    auto go = [&](auto kernel) {
-      static bool done = false;
-      if (!done) {
-        check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  160 * 1024 - 1024),
-              "hipFuncSetAttribute");
-        done = true;
-      }
-      hipLaunchKernelGGL(kernel, dim3(n * KV * ((G + GH - 1) / GH)), dim3(kAttnThreads), lds, s, q, q_stride, out, out_stride, G,
-                         scale, a, seq, n_keys, anc_off, anc, n, KV, nk_pad, anc_cap, xq, xq_stride);
+    auto go = [&]<int N>() {
+      allow_lds<k_attention_grp<N>>(kLdsLimit);
+      hipLaunchKernelGGL(k_attention_grp<N>, dim3(n * KV * ((G + N - 1) / N)), dim3(kAttnThreads), lds, s, q, q_stride,
+                         out, out_stride, G, scale, a, seq, n_keys, anc_off, anc, n, KV, nk_pad, anc_cap, xq, xq_stride);
     };
     switch (GH) {
-      case 1: go(k_attention_grp<1>); break;
-      case 2: go(k_attention_grp<2>); break;
-      case 3: go(k_attention_grp<3>); break;
-      case 4: go(k_attention_grp<4>); break;
-      default: go(k_attention_grp<5>); break;
+      case 1: go.template operator()<1>(); break;
+      case 2: go.template operator()<2>(); break;
+      case 3: go.template operator()<3>(); break;
+      case 4: go.template operator()<4>(); break;
+      default: go.template operator()<5>(); break;
     }
   } else if (G <= 16 && (D == 64 || D == 128 || D == 256) && aligned) {
     const int tile = D == 64 ? AttnTile<64>::tile : D == 128 ? AttnTile<128>::tile : AttnTile<256>::tile;
     const int nk_pad = attn_keys_pad(max_keys);
     const size_t lds = attn_lds_bytes(tile, D, nk_pad);
-    auto attr = [&](auto kernel, bool& done) {
-      if (!done) {
-        check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  160 * 1024 - 1024),
-              "hipFuncSetAttribute");
-        done = true;
-      }
-    };
-    if (lds <= 160 * 1024 - 1024) {
-      auto go = [&](auto kernel) {
-        static bool done = false;
-        attr(kernel, done);
-        hipLaunchKernelGGL(kernel, dim3(n * H), dim3(kAttnThreads), lds, s, q, q_stride, out, out_stride, G, scale, a,
-                           seq, n_keys, anc_off, anc, n, H, xq, xq_stride);
-      };
+    // D and the K rows' order as constants
+    auto with_form = [&](auto go) {
       if (D == 64)
-        a.k_perm ? go(k_attention<64, true>) : go(k_attention<64, false>);
+        a.k_perm ? go.template operator()<64, true>() : go.template operator()<64, false>();
       else if (D == 128)
-        a.k_perm ? go(k_attention<128, true>) : go(k_attention<128, false>);
+        a.k_perm ? go.template operator()<128, true>() : go.template operator()<128, false>();
       else
-        a.k_perm ? go(k_attention<256, true>) : go(k_attention<256, false>);
+        a.k_perm ? go.template operator()<256, true>() : go.template operator()<256, false>();
+    };
+    if (lds <= kLdsLimit) {
+      with_form([&]<int DD, bool PERM>() {
+        allow_lds<k_attention<DD, PERM>>(kLdsLimit);
+        hipLaunchKernelGGL((k_attention<DD, PERM>), dim3(n * H), dim3(kAttnThreads), lds, s, q, q_stride, out, out_stride,
+                           G, scale, a, seq, n_keys, anc_off, anc, n, H, xq, xq_stride);
+      });
     } else {
       // More keys than LDS holds: scores and coefficients in global slots of the caller's scratch.
       const size_t slot = 2 * (size_t)nk_pad * sizeof(float);
@@ -1518,19 +1496,12 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
       require(scratch && slots >= 1, "attention: too many keys for the scratch buffer (mk_reserve_scratch)");
       const int chunk = D == 64 ? AttnTile<64>::chunk : D == 128 ? AttnTile<128>::chunk : AttnTile<256>::chunk;
       const size_t lds_long = 2 * (size_t)tile + 4 * ((size_t)D + 4 * (size_t)chunk);
-      auto go = [&](auto kernel) {
-        static bool done = false;
-        attr(kernel, done);
-        hipLaunchKernelGGL(kernel, dim3(slots), dim3(kAttnThreads), lds_long, s, q, q_stride, out, out_stride, G,
-                           scale, a, seq, n_keys, anc_off, anc, n, H, static_cast<float*>(scratch), nk_pad, xq,
-                           xq_stride);
-      };
-      if (D == 64)
-        a.k_perm ? go(k_attention_long<64, true>) : go(k_attention_long<64, false>);
-      else if (D == 128)
-        a.k_perm ? go(k_attention_long<128, true>) : go(k_attention_long<128, false>);
-      else
-        a.k_perm ? go(k_attention_long<256, true>) : go(k_attention_long<256, false>);
+      with_form([&]<int DD, bool PERM>() {
+        allow_lds<k_attention_long<DD, PERM>>(kLdsLimit);
+        hipLaunchKernelGGL((k_attention_long<DD, PERM>), dim3(slots), dim3(kAttnThreads), lds_long, s, q, q_stride, out,
+                           out_stride, G, scale, a, seq, n_keys, anc_off, anc, n, H, static_cast<float*>(scratch), nk_pad,
+                           xq, xq_stride);
+      });
     }
   } else {
     const size_t lds = (size_t)(D + 2 * (size_t)max_keys) * sizeof(float);

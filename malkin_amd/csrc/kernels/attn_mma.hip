@@ -373,13 +373,7 @@ void attention_mma(hipStream_t s, const float* q, int64_t q_stride, float* out, 
                    int64_t xq_stride) {
   const int TQ = kRows / G, max_pad = pad64(max_keys);
   auto go = [&]<bool LONG>(int nk_pad) {
-    static bool attr = false;  // per instantiation
-    if (!attr) {
-      check(hipFuncSetAttribute(reinterpret_cast<const void*>(k_attention_mma<LONG>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds),
-            "hipFuncSetAttribute");
-      attr = true;
-    }
+    allow_lds<k_attention_mma<LONG>>((int)kLds);
     hipLaunchKernelGGL(k_attention_mma<LONG>, dim3(((n + TQ - 1) / TQ) * KV), dim3(kThreads), mma_lds_bytes(nk_pad), s, q, q_stride,
                        out, out_stride, G, scale, a, seq, n_keys, n, KV, max_pad, xq, xq_stride);
   };

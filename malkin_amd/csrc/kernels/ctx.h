@@ -53,6 +53,16 @@ inline int device_cus() {
   return n;
 }
 
+// Allows launches of Kernel up to `bytes` of dynamic LDS (past the default 64 KB); once per kernel, from any thread.
+template <auto Kernel>
+void allow_lds(int bytes) {
+  static const bool set = (check(hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, bytes),
+                                 "hipFuncSetAttribute"),
+                           true);
+  (void)set;
+}
+
 template <typename F>
 int guard(F&& f) {
   try {

@@ -752,14 +752,9 @@ void decode_layers(hipStream_t s, const void* dev_args, const DecodeDims& d, int
   const size_t lds = std::max(gemv_lds_bytes(max_cols, d.E, ring), dec_lds_bytes(d.D, attn_keys_pad(max_keys)));
   const int cus = device_cus();
   const DecodeArgs* P = static_cast<const DecodeArgs*>(dev_args);
-  auto go = [&](auto kernel) {
-    static bool attr = false;
-    if (!attr) {
-      check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                160 * 1024 - kStaticLds),
-            "hipFuncSetAttribute");
-      attr = true;
-    }
+  auto go = [&]<int SLOTS, int RING>() {
+    constexpr auto kernel = k_decode_layers<128, SLOTS, RING>;
+    allow_lds<kernel>(160 * 1024 - kStaticLds);
     hipFuncAttributes fa{};
     check(hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(kernel)), "hipFuncGetAttributes");
     require(fa.sharedSizeBytes <= (size_t)kStaticLds, "decode_layers: static LDS above its bound");
@@ -771,15 +766,15 @@ void decode_layers(hipStream_t s, const void* dev_args, const DecodeDims& d, int
     hipLaunchKernelGGL(kernel, dim3(cus), dim3(kDT), lds, s, P, l0, l1);
   };
   const int slots = dec_slots(d.D, max_keys, true, kDT);
-  auto pick = [&](auto k4, auto k3) { ring == 4 ? go(k4) : go(k3); };
+  auto pick = [&]<int SLOTS>() { ring == 4 ? go.template operator()<SLOTS, 4>() : go.template operator()<SLOTS, 3>(); };
   if (slots <= 2)
-    pick(k_decode_layers<128, 2, 4>, k_decode_layers<128, 2, 3>);
+    pick.template operator()<2>();
   else if (slots <= 4)
-    pick(k_decode_layers<128, 4, 4>, k_decode_layers<128, 4, 3>);
+    pick.template operator()<4>();
   else if (slots <= 6)
-    pick(k_decode_layers<128, 6, 4>, k_decode_layers<128, 6, 3>);
+    pick.template operator()<6>();
   else
-    pick(k_decode_layers<128, kMaxSlots, 4>, k_decode_layers<128, kMaxSlots, 3>);
+    pick.template operator()<kMaxSlots>();
   check_launch("decode_layers");
 }
 
