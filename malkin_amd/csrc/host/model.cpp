@@ -561,6 +561,7 @@ void Model::finish_layout() {
   std::vector<int32_t> seqs(L.seq);
   std::sort(seqs.begin(), seqs.end());
   L.distinct_seqs = std::adjacent_find(seqs.begin(), seqs.end()) == seqs.end();
+  L.walks = mk::attention_walks(L.seq.data(), L.n, cfg_.n_head / cfg_.n_head_kv);
 }
 
 void Model::check_ids() {
@@ -656,12 +657,9 @@ void Model::run() {
       ck(mk_qk_norm_rope_kv(ctx_, qkv, qkv + static_cast<int64_t>(H) * D, qkv + static_cast<int64_t>(H + KV) * D, QKV,
                             n, H, norms + 2 * E, norms + 2 * E + D, c.rms_eps, rope_cos_.as<float>(),
                             rope_sin_.as<float>(), d_rpos_, d_seq_, d_kv_row_, &kv, il));
-      if (wo_f32)
-        ck(mk_attention(ctx_, qkv, QKV, att, static_cast<int64_t>(H) * D, n, H, &kv, il, d_seq_, d_n_keys_,
-                        lay_.tree ? d_extra_at_ : nullptr, d_extra_, lay_.max_keys));
-      else
-        ck(mk_attention_q8(ctx_, qkv, QKV, att, static_cast<int64_t>(H) * D, n, H, &kv, il, d_seq_, d_n_keys_,
-                           lay_.tree ? d_extra_at_ : nullptr, d_extra_, lay_.max_keys, xq));
+      ck(mk::attention_batch(ctx_, qkv, QKV, att, static_cast<int64_t>(H) * D, n, H, &kv, il, d_seq_, d_n_keys_,
+                             lay_.tree ? d_extra_at_ : nullptr, d_extra_, lay_.max_keys, wo_f32 ? nullptr : xq,
+                             &lay_.walks));
     } else {
       ck(rc);
     }
@@ -755,8 +753,8 @@ void Model::run_row_layer(const Layer& L, int il) {
   ck(mk_qk_norm_rope_kv(ctx_, qkv, qkv + HD, qkv + HD + static_cast<int64_t>(KV) * D, QKV, n, H, norms + 2 * E,
                         norms + 2 * E + D, c.rms_eps, rope_cos_.as<float>(), rope_sin_.as<float>(), d_rpos_, d_seq_,
                         d_kv_row_, &kv_, il));
-  ck(mk_attention_q8(ctx_, qkv, QKV, att, HD, n, H, &kv_, il, d_seq_, d_n_keys_,
-                     lay_.tree ? d_extra_at_ : nullptr, d_extra_, lay_.max_keys, xq));  // att and its BlockQ8 rows
+  ck(mk::attention_batch(ctx_, qkv, QKV, att, HD, n, H, &kv_, il, d_seq_, d_n_keys_, lay_.tree ? d_extra_at_ : nullptr,
+                         d_extra_, lay_.max_keys, xq, &lay_.walks));  // att and its BlockQ8 rows
   single(L.wo, att, HD, x, E);  // x += attn_output(att)
   ck(mk_rmsnorm_rows(ctx_, x, nullptr, norms + E, n, E, c.rms_eps, h));
   ck(mk_quantize_q8(ctx_, h, n, E, xq));

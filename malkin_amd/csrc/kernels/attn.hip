@@ -547,7 +547,9 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention_long(const float* __
                                                                  const int32_t* __restrict__ anc_off,
                                                                  const int32_t* __restrict__ anc, int n, int H,
                                                                  float* __restrict__ gsc, int gcap,
-                                                                 BlockQ8* __restrict__ xq, int64_t xq_stride) {
+                                                                 BlockQ8* __restrict__ xq, int64_t xq_stride,
+                                                                 const int32_t* __restrict__ route) {
+  if (route && *route == kRouteMma) return;
   float* slot = gsc + (size_t)blockIdx.x * 2 * (size_t)gcap;
   for (int pair = (int)blockIdx.x; pair < n * H; pair += (int)gridDim.x) {
     __syncthreads();  // the previous pair's LDS and slot are no longer read
@@ -588,7 +590,8 @@ __host__ __device__ constexpr size_t grp_lds_bytes(int GH, int nk_pad, int anc_c
   return 2 * (size_t)GrpCfg<2>::tile + 4 * ((size_t)GH * 128 + 2 * (size_t)GH * nk_pad + (size_t)anc_cap);
 }
 
-template <int GH>
+// ROUTED: the workgroups leave at once if *route sends the batch to attention_mma.
+template <int GH, bool ROUTED>
 __global__ __launch_bounds__(kAttnThreads) void k_attention_grp(const float* __restrict__ q, int64_t q_stride,
                                                                 float* __restrict__ out, int64_t out_stride, int G,
                                                                 float scale, AttnAddr a,
@@ -597,9 +600,11 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention_grp(const float* __r
                                                                 const int32_t* __restrict__ anc_off,
                                                                 const int32_t* __restrict__ anc, int n, int KV,
                                                                 int nk_pad, int anc_cap, BlockQ8* __restrict__ xq,
-                                                                int64_t xq_stride) {
+                                                                int64_t xq_stride, const int32_t* __restrict__ route) {
   using C = GrpCfg<GH>;
   constexpr int D = C::D, DC = C::DC, CK = C::CK, VS = C::VS;
+  if constexpr (ROUTED)
+    if (*route == kRouteMma) return;
   const int tid = threadIdx.x;
   // (group, token, head subset) numbered group-major; XCD x (workgroups x, x + 8, ...) takes a contiguous run, so a
   // group's K/V rows are read into one XCD's L2.
@@ -902,8 +907,44 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention_grp(const float* __r
     float* o = out + t * out_stride + (int64_t)(hfirst + hb) * D + d;
 #pragma unroll
     for (int k = 0; k < C::h0; ++k)
-      if (k < nh && hfirst + hb + k >= hout) put_out(o + k * D - d, xq, t * xq_stride, (hfirst + hb + k) * D, d, acc[k] * inv_s[hb + k]);
+      if (k < nh && hfirst + hb + k >= hout)
+        put_out(o + k * D - d, xq, t * xq_stride, (hfirst + hb + k) * D, d, acc[k] * inv_s[hb + k]);
   }
+}
+
+// Whether attention_mma takes a plain batch of rows longer than its LDS holds: its walks, in rounds of the CUs (one workgroup
+// per KV head and token block, one walk after the other), cost no more than `rest`, the kernel that takes the tokens
+// otherwise (rest_cost). Units of 1/200 of a walk. Where about every block has as many walks as the longest, a round lasts
+// that long; a few long blocks fill the others' rounds in part.
+__host__ __device__ inline bool mma_pays(const AttnWalks& w, int blocks, int KV, int cus, int rest) {
+  auto rounds = [&](int64_t n) { return (int)((n * KV + cus - 1) / cus); };
+  const int even = rounds(w.all), full = min(even + w.most - 1, rounds(blocks) * w.most);
+  const int r = 4 * (int64_t)w.all >= 3 * (int64_t)blocks * w.most ? full : min(full, max(even, w.most) + (w.most - 1) / 2);
+  return 200 * (int64_t)r <= rest;
+}
+
+// Whether a plain batch's walks pay, for callers whose sequences only the device knows. 16 lanes per token block.
+__global__ __launch_bounds__(1024) void k_attention_route(const int32_t* __restrict__ seqs, int n, int TQ, int KV, int cus,
+                                                          int rest, int32_t* __restrict__ route) {
+  __shared__ int all_s, most_s;
+  if (threadIdx.x == 0) all_s = most_s = 0;
+  __syncthreads();
+  const int l = threadIdx.x & 15, row = threadIdx.x & 48, nblk = (n + TQ - 1) / TQ;
+  for (int b0 = 0; b0 < nblk; b0 += 64) {
+    const int b = b0 + (int)(threadIdx.x >> 4);
+    const bool in = b < nblk && l < TQ && b * TQ + l < n;
+    const int s = in ? seqs[b * TQ + l] : -1;
+    int again = 0;  // a lane of the block below this one holds the same sequence
+#pragma unroll
+    for (int k = 0; k < 15; ++k) again |= (int)(k < l) & (int)(__shfl(s, k, 16) == s);
+    const int c = __popcll(__ballot(in && !again) >> row & 0xFFFF);
+    if (l == 0 && c > 0) {
+      atomicAdd(&all_s, c);
+      atomicMax(&most_s, c);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) *route = mma_pays({all_s, most_s}, nblk, KV, cus, rest) ? kRouteMma : 0;
 }
 
 // Attention of many query rows at once (prefill and other long plain batches) for the head size that attn_mma.hip does
@@ -1425,26 +1466,63 @@ int grp_heads(int n, int H, int G, int D, const AttnAddr& a, const int32_t* anc_
   return grp_lds_bytes(1, nk_pad, anc_cap) <= limit ? 1 : 0;
 }
 
+// What the batch costs without attention_mma, in 1/200 of a walk of its workgroups over the keys: rounds of the grouped kernel
+// (GH heads a workgroup; 52, 65, 72 and 97 us at 1, 2, 4 and 5 heads where a walk takes 177, at 4000 keys; the same shares
+// from 2000 to 8000), past that one's keys of k_attention_long (as much as a walk).
+int rest_cost(int n, int KV, int G, int GH) {
+  const int64_t cus = device_cus(), wgs = (int64_t)n * KV * (GH > 0 ? (G + GH - 1) / GH : G);
+  return (int)std::min<int64_t>(INT32_MAX, (wgs + cus - 1) / cus * (GH > 0 ? 47 + 12 * GH : 190));
+}
+
+template <typename F>
+void with_heads(int GH, F go) {
+  switch (GH) {
+    case 1: go.template operator()<1>(); break;
+    case 2: go.template operator()<2>(); break;
+    case 3: go.template operator()<3>(); break;
+    case 4: go.template operator()<4>(); break;
+    default: go.template operator()<5>(); break;
+  }
+}
+
 void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int64_t out_stride, int n, int H, int KV,
                int D, float scale, const AttnAddr& a, const int32_t* seq, const int32_t* n_keys,
-               const int32_t* anc_off, const int32_t* anc, int max_keys, void* scratch, size_t scratch_bytes,
-               BlockQ8* xq, int64_t xq_stride) {
+               const int32_t* anc_off, const int32_t* anc, int max_keys, int n_seq, const AttnWalks* walks, int32_t* route,
+               void* scratch, size_t scratch_bytes, BlockQ8* xq, int64_t xq_stride) {
   if (n <= 0) return;
   require(D % 16 == 0 && D <= 256 && H % KV == 0 && max_keys > 0, "attention: unsupported head layout");
   require(!xq || D % 32 == 0, "attention: Q8 rows need head_dim % 32 == 0");
   const int G = H / KV;
   const bool aligned = attn_aligned(a);
-  // Many plain tokens on the matrix cores. Rows longer than its LDS holds run their scores twice, which pays where the
-  // grouped kernel (one workgroup per token and KV group) needs more than two rounds of the CUs: 32 heads over 2000 keys
-  // at 32 / 64 / 128 / 256 tokens 47 / 96 / 189 / 380 us grouped, 93 / 98 / 105 / 207 here. (Past the grouped kernel's
-  // keys the caller's scratch must hold a row all the same: such calls have always needed it.)
-  if (!anc_off && n >= kRowsMinTokens && attention_mma_ok(G, D, a) &&
-      (attention_mma_whole(max_keys) ||
-       ((int64_t)n * KV > 2 * device_cus() &&
-        (grp_heads(n, H, G, D, a, anc_off, max_keys) > 0 ||
-         (scratch && scratch_bytes >= 2 * (size_t)attn_keys_pad(max_keys) * sizeof(float)))))) {
-    attention_mma(s, q, q_stride, out, out_stride, n, G, KV, scale, a, seq, n_keys, max_keys, xq, xq_stride);
-  } else if (!anc_off && n >= kRowsMinTokens && G <= 16 && D == 64 && a.k_perm && aligned &&
+  const int GH = grp_heads(n, H, G, D, a, anc_off, max_keys);
+  // Many plain tokens on the matrix cores: always where a row's scores fit LDS. Longer rows, whose scores run twice, where
+  // the batch takes more than two rounds of the CUs otherwise and its walks pay (mma_pays); where only the device knows
+  // the sequences and they matter, it decides: both kernels are launched and one of them leaves at once (4 to 9 us). Measured at
+  // 32 heads over 8 KV heads, the grouped kernel / this, us: 128 tokens of one sequence over 2000 keys 169 / 92, of 64
+  // sequences 171 / 187, of 128 180 / 366; 128 tokens over 3000 keys, where a group's heads take workgroups of their own,
+  // 645 / 133, 534 / 279 and 541 / 500; 8 heads over 8 KV heads, 80 tokens of one sequence over 4000 keys 159 / 177.
+  // (Past the grouped kernel's keys the caller's scratch must hold a row all the same: such calls have always needed it.)
+  const int32_t* routed = nullptr;
+  if (!anc_off && n >= kRowsMinTokens && attention_mma_ok(G, D, a)) {
+    bool mma = attention_mma_whole(max_keys);
+    if (!mma && (int64_t)n * KV > 2 * device_cus() &&
+        (GH > 0 || (scratch && scratch_bytes >= 2 * (size_t)attn_keys_pad(max_keys) * sizeof(float)))) {
+      const int TQ = kRowsMax / G, nblk = (n + TQ - 1) / TQ, cus = device_cus();
+      const int rest = rest_cost(n, KV, G, GH);
+      // One sequence a block at best; at worst every token of a block its own (or as many as the cache has).
+      const AttnWalks best{nblk, 1}, worst{std::min<int>(n, nblk * std::min(TQ, n_seq)), std::min({TQ, n_seq, n})};
+      mma = mma_pays(walks ? *walks : best, nblk, KV, cus, rest);
+      if (mma && !walks && !mma_pays(worst, nblk, KV, cus, rest)) {
+        hipLaunchKernelGGL(k_attention_route, dim3(1), dim3(1024), 0, s, seq, n, TQ, KV, cus, rest, route);
+        routed = route;
+      }
+    }
+    if (mma) {
+      attention_mma(s, q, q_stride, out, out_stride, n, G, KV, scale, a, seq, n_keys, max_keys, xq, xq_stride, routed);
+      if (!routed) return;
+    }
+  }
+  if (!anc_off && n >= kRowsMinTokens && G <= 16 && D == 64 && a.k_perm && aligned &&
              rows_lds_bytes(D, attn_keys_pad(max_keys)) <= 160 * 1024 - 1024) {
     const int nk_pad = attn_keys_pad(max_keys), TQ = kRowsMax / G;
     allow_lds<k_attention_rows<64>>(kLdsLimit);
@@ -1453,23 +1531,17 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
   } else if (!anc_off && dec_ok(G, D, a, max_keys)) {
     launch_dec<false>(s, q, q_stride, out, out_stride, n, H, D, G, scale, a, seq, n_keys, max_keys, DecFuse{}, xq,
                       xq_stride);
-  } else if (grp_heads(n, H, G, D, a, anc_off, max_keys) > 0) {
+  } else if (GH > 0) {
     // Grouped workgroups (trees, keys past the decode kernel's LDS).
-    const int GH = grp_heads(n, H, G, D, a, anc_off, max_keys);
     const int nk_pad = attn_keys_pad(max_keys), anc_cap = anc_off ? std::min(n, nk_pad) : 0;
     const size_t lds = grp_lds_bytes(GH, nk_pad, anc_cap);
-    auto go = [&]<int N>() {
-      allow_lds<k_attention_grp<N>>(kLdsLimit);
-      hipLaunchKernelGGL(k_attention_grp<N>, dim3(n * KV * ((G + N - 1) / N)), dim3(kAttnThreads), lds, s, q, q_stride,
-                         out, out_stride, G, scale, a, seq, n_keys, anc_off, anc, n, KV, nk_pad, anc_cap, xq, xq_stride);
+    auto go = [&]<int N, bool ROUTED>() {
+      allow_lds<k_attention_grp<N, ROUTED>>(kLdsLimit);
+      hipLaunchKernelGGL((k_attention_grp<N, ROUTED>), dim3(n * KV * ((G + N - 1) / N)), dim3(kAttnThreads), lds, s, q,
+                         q_stride, out, out_stride, G, scale, a, seq, n_keys, anc_off, anc, n, KV, nk_pad, anc_cap, xq,
+                         xq_stride, routed);
     };
-    switch (GH) {
-      case 1: go.template operator()<1>(); break;
-      case 2: go.template operator()<2>(); break;
-      case 3: go.template operator()<3>(); break;
-      case 4: go.template operator()<4>(); break;
-      default: go.template operator()<5>(); break;
-    }
+    with_heads(GH, [&]<int N>() { routed ? go.template operator()<N, true>() : go.template operator()<N, false>(); });
   } else if (G <= 16 && (D == 64 || D == 128 || D == 256) && aligned) {
     const int tile = D == 64 ? AttnTile<64>::tile : D == 128 ? AttnTile<128>::tile : AttnTile<256>::tile;
     const int nk_pad = attn_keys_pad(max_keys);
@@ -1500,7 +1572,7 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
         allow_lds<k_attention_long<DD, PERM>>(kLdsLimit);
         hipLaunchKernelGGL((k_attention_long<DD, PERM>), dim3(slots), dim3(kAttnThreads), lds_long, s, q, q_stride, out,
                            out_stride, G, scale, a, seq, n_keys, anc_off, anc, n, H, static_cast<float*>(scratch), nk_pad,
-                           xq, xq_stride);
+                           xq, xq_stride, routed);
       });
     }
   } else {

@@ -18,7 +18,7 @@
 // Scores and v scales of a 16-key group lie in LDS in the order lane q of the P.V reads them (key 4 s + q at 4 q + s).
 // Rows longer than LDS holds (LONG) take two passes: the maxima first, then the scores again, kChunk keys at a time, each
 // chunk's sums and P.V continuing the last one's. Tokens of a block that belong to different sequences are handled
-// one sequence at a time.
+// one sequence at a time, each in a walk over that sequence's keys.
 //
 // What bounds it: fp32 MFMAs and vector instructions share a SIMD's issue (measured: they do not overlap), so a 16-key
 // score tile costs 32 x 32 cycles of MFMA and about 150 vector instructions (transpose, conversions, the trees), and
@@ -80,7 +80,9 @@ __global__ __launch_bounds__(kThreads) void k_attention_mma(const float* __restr
                                                             float* __restrict__ out, int64_t out_stride, int G,
                                                             float scale, AttnAddr a, const int32_t* __restrict__ seqs,
                                                             const int32_t* __restrict__ n_keys, int n, int KV,
-                                                            int max_pad, BlockQ8* __restrict__ xq, int64_t xq_stride) {
+                                                            int max_pad, BlockQ8* __restrict__ xq, int64_t xq_stride,
+                                                            const int32_t* __restrict__ route) {
+  if (LONG && route && *route != kRouteMma) return;
   const int nk_pad = LONG ? kChunk : max_pad;  // keys held in LDS
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lq = lane >> 4;
@@ -370,12 +372,12 @@ bool attention_mma_whole(int max_keys) { return mma_lds_bytes(pad64(max_keys)) <
 
 void attention_mma(hipStream_t s, const float* q, int64_t q_stride, float* out, int64_t out_stride, int n, int G, int KV,
                    float scale, const AttnAddr& a, const int32_t* seq, const int32_t* n_keys, int max_keys, BlockQ8* xq,
-                   int64_t xq_stride) {
+                   int64_t xq_stride, const int32_t* route) {
   const int TQ = kRows / G, max_pad = pad64(max_keys);
   auto go = [&]<bool LONG>(int nk_pad) {
     allow_lds<k_attention_mma<LONG>>((int)kLds);
     hipLaunchKernelGGL(k_attention_mma<LONG>, dim3(((n + TQ - 1) / TQ) * KV), dim3(kThreads), mma_lds_bytes(nk_pad), s, q, q_stride,
-                       out, out_stride, G, scale, a, seq, n_keys, n, KV, max_pad, xq, xq_stride);
+                       out, out_stride, G, scale, a, seq, n_keys, n, KV, max_pad, xq, xq_stride, route);
   };
   if (attention_mma_whole(max_keys))
     go.template operator()<false>(max_pad);

@@ -1,6 +1,7 @@
 // extern "C" layer of include/malkin_hip.h over the internal launchers.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdarg>
@@ -348,7 +349,7 @@ int mk_attend_gqa(mk_ctx* c, const float* q, int G, int D, const int8_t* k, cons
     mk::AttnAddr a{k, v, reinterpret_cast<const char*>(k) + soff, reinterpret_cast<const char*>(v) + soff,
                    0, 0, (int64_t)stride, 0, 0, (int64_t)stride, 0};
     mk::attention(c->stream, q, (int64_t)G * D, out, (int64_t)G * D, 1, G, 1, D, scale, a, dm, dm + 1,
-                  ne > 0 ? dm + 2 : nullptr, extra, n + ne, c->scratch, c->scratch_bytes);
+                  ne > 0 ? dm + 2 : nullptr, extra, n + ne, 1, nullptr, c->meta + 4, c->scratch, c->scratch_bytes);
   });
 }
 
@@ -373,7 +374,8 @@ namespace {
 
 void attention_rows(mk_ctx* c, const float* q, int64_t q_stride, float* out, int64_t out_stride, int n, int n_head,
                     const mk_kv_cache* kv, int layer, const int32_t* seq, const int32_t* n_keys,
-                    const int32_t* anc_off, const int32_t* anc, int max_keys, void* xq) {
+                    const int32_t* anc_off, const int32_t* anc, int max_keys, void* xq,
+                    const mk::AttnWalks* walks = nullptr) {
   const mk::KvLayer L = kv_layer(kv, layer);
   const int D = kv->head_dim;
   const int64_t rows = (int64_t)kv->n_ctx;
@@ -382,7 +384,8 @@ void attention_rows(mk_ctx* c, const float* q, int64_t q_stride, float* out, int
                  (int64_t)kv->n_head_kv * rows * 4, rows * 4, 4, 1};
   const float scale = 1.0f / std::sqrt(static_cast<float>(D));  // model.cpp:208
   mk::attention(c->stream, q, q_stride, out, out_stride, n, n_head, kv->n_head_kv, D, scale, a, seq, n_keys, anc_off,
-                anc, max_keys, c->scratch, c->scratch_bytes, static_cast<mk::BlockQ8*>(xq), (int64_t)n_head * D / 32);
+                anc, max_keys, kv->n_seq, walks, c->meta + 4, c->scratch, c->scratch_bytes,
+                static_cast<mk::BlockQ8*>(xq), (int64_t)n_head * D / 32);
 }
 
 void attention_decode(mk_ctx* c, const float* qkv, int64_t stride, int n, int n_head, const float* q_norm,
@@ -403,6 +406,32 @@ void attention_decode(mk_ctx* c, const float* qkv, int64_t stride, int n, int n_
 }
 
 }  // namespace
+
+}  // extern "C"
+
+namespace mk {
+AttnWalks attention_walks(const int32_t* host_seq, int n, int G) {
+  AttnWalks w;
+  const int tq = 16 / std::min(std::max(G, 1), 16);
+  for (int t0 = 0; t0 < n; t0 += tq) {
+    int c = 0;
+    for (int t = t0; t < std::min(t0 + tq, n); ++t) c += std::find(host_seq + t0, host_seq + t, host_seq[t]) == host_seq + t;
+    w.all += c;
+    w.most = std::max(w.most, c);
+  }
+  return w;
+}
+
+int attention_batch(mk_ctx* c, const float* q, int64_t q_stride, float* out, int64_t out_stride, int n, int n_head,
+                    const mk_kv_cache* kv, int layer, const int32_t* seq, const int32_t* n_keys, const int32_t* anc_off,
+                    const int32_t* anc, int max_keys, void* xq, const AttnWalks* walks) {
+  return guard([&] {
+    attention_rows(c, q, q_stride, out, out_stride, n, n_head, kv, layer, seq, n_keys, anc_off, anc, max_keys, xq, walks);
+  });
+}
+}  // namespace mk
+
+extern "C" {
 
 int mk_attention_q8(mk_ctx* c, const float* q, int64_t q_stride, float* out, int64_t out_stride, int n, int n_head,
                     const mk_kv_cache* kv, int layer, const int32_t* seq, const int32_t* n_keys,

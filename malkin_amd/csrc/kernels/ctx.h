@@ -18,7 +18,8 @@ struct mk_ctx {
   char name[64] = {0};
   void* scratch = nullptr;  // per-context device scratch (partial reductions), allocated once at init
   size_t scratch_bytes = 0;
-  int32_t* meta = nullptr;  // 64 bytes of per-call metadata (mk_attend_gqa's token layout), allocated at init
+  int32_t* meta = nullptr;  // 64 bytes of per-call metadata (words 0..3: mk_attend_gqa's token layout, 4: attention's
+                            // route), allocated at init
 };
 
 namespace mk {
@@ -62,6 +63,18 @@ void allow_lds(int bytes) {
                            true);
   (void)set;
 }
+
+// The walks over a sequence's keys that attention on the matrix cores makes for a plain batch, per KV head: for each block
+// of 16 / G consecutive tokens one per sequence among them. All blocks' and the most of one block.
+struct AttnWalks {
+  int all = 0, most = 0;
+};
+AttnWalks attention_walks(const int32_t* host_seq, int n, int G);
+
+// mk_attention (xq NULL) and mk_attention_q8 for a caller that knows the batch's walks on the host.
+int attention_batch(mk_ctx* ctx, const float* q, int64_t q_stride, float* out, int64_t out_stride, int n, int n_head,
+                    const mk_kv_cache* kv, int layer, const int32_t* seq, const int32_t* n_keys, const int32_t* anc_off,
+                    const int32_t* anc, int max_keys, void* xq, const AttnWalks* walks);
 
 template <typename F>
 int guard(F&& f) {

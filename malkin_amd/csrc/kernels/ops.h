@@ -126,19 +126,24 @@ __host__ __device__ constexpr int kv_perm(int e, int DC) { return DC * (e & 15) 
 // q [n][H*D] (token stride q_stride floats), out [n][H*D] (stride out_stride). Per token t: keys rows
 // 0..n_keys[t]-1 of sequence seq[t], then anc[anc_off[t] .. anc_off[t+1]) when anc_off is non-null. Rows with more
 // keys than one workgroup's LDS holds keep their scores in `scratch` (attention_scratch_bytes of it for full speed;
-// a smaller scratch runs fewer workgroups at a time; one without room for a single row fails).
+// a smaller scratch runs fewer workgroups at a time; one without room for a single row fails). walks: those of the batch,
+// where the host knows seq; else the device finds out where it matters, into *route (a device word of the context; n_seq,
+// the cache's sequences, bounds the batch's).
+struct AttnWalks;             // ctx.h
+constexpr int kRouteMma = 1;  // *route: every token to attention_mma (0: none)
 void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int64_t out_stride, int n, int H, int KV,
                int D, float scale,
                const AttnAddr& a, const int32_t* seq, const int32_t* n_keys, const int32_t* anc_off,
-               const int32_t* anc, int max_keys, void* scratch, size_t scratch_bytes, BlockQ8* xq = nullptr,
-               int64_t xq_stride = 0);
+               const int32_t* anc, int max_keys, int n_seq, const AttnWalks* walks, int32_t* route, void* scratch,
+               size_t scratch_bytes, BlockQ8* xq = nullptr, int64_t xq_stride = 0);
 // Plain batches of many tokens at head_dim 128 over the permuted device cache (attn_mma.hip); attention()'s choice from
-// 16 tokens on.
+// 16 tokens on.  With route (only
+// where a row is longer than LDS holds) it does nothing unless *route is kRouteMma.
 bool attention_mma_ok(int G, int D, const AttnAddr& a);
 bool attention_mma_whole(int max_keys);  // a row's scores fit LDS (else they are computed twice)
 void attention_mma(hipStream_t s, const float* q, int64_t q_stride, float* out, int64_t out_stride, int n, int G, int KV,
                    float scale, const AttnAddr& a, const int32_t* seq, const int32_t* n_keys, int max_keys, BlockQ8* xq,
-                   int64_t xq_stride);
+                   int64_t xq_stride, const int32_t* route);
 // Scratch the attention of `pairs` (token, head) pairs over max_keys keys uses (0: none).
 size_t attention_scratch_bytes(int D, int max_keys, int pairs);
 
