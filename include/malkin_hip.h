@@ -285,7 +285,8 @@ int mk_penalize(mk_ctx* ctx, float* logits, int64_t stride, const int32_t* rows,
 /* The top-k cut of Sampler::distribution (sampler.cpp:32-36, std::partial_sort by value): per row the k largest
    logits, highest first, into values / ids [n_rows][k]. k = 1..1024 and at most n_vocab. Equal logits are ordered
    by lower id (the reference leaves their order unspecified). Rows past 8192 logits are selected from in slices whose
-   candidates go through the context's scratch (no allocation). */
+   candidates go through memory that the context holds for it from mk_init on (no allocation; a captured graph stays
+   valid whatever mk_reserve_scratch does later). */
 int mk_topk(mk_ctx* ctx, const float* logits, int64_t stride, const int32_t* rows, int n_rows, int n_vocab, int k,
             float* values, int32_t* ids);
 /* Per-row parameters of mk_sample_cut: candidates k (<= 0: the whole vocabulary) and the request's temperature

@@ -76,6 +76,7 @@ int mk_init(int device, mk_ctx** out) {
     check(hipEventCreate(&c->ev1), "hipEventCreate");
     c->scratch_bytes = 1 << 20;
     check(hipMalloc(&c->scratch, c->scratch_bytes), "hipMalloc");
+    check(hipMalloc(&c->topk_cand, mk::topk_workspace()), "hipMalloc");
     check(hipMalloc(&c->meta, 64), "hipMalloc");
     *out = c;
   });
@@ -90,6 +91,7 @@ int mk_destroy(mk_ctx* c) {
     (void)hipEventDestroy(c->ev1);
     (void)hipStreamDestroy(c->stream);
     (void)hipFree(c->scratch);
+    (void)hipFree(c->topk_cand);
     (void)hipFree(c->meta);
     delete c;
   });
@@ -511,7 +513,7 @@ int mk_topk(mk_ctx* c, const float* logits, int64_t stride, const int32_t* rows,
             float* values, int32_t* ids) {
   return guard([&] {
     require(logits && values && ids && n_rows >= 0 && n_vocab > 0 && stride >= n_vocab, "topk: bad arguments");
-    mk::topk(c->stream, logits, stride, rows, n_rows, n_vocab, k, values, ids, c->scratch, c->scratch_bytes);
+    mk::topk(c->stream, logits, stride, rows, n_rows, n_vocab, k, values, ids, c->topk_cand);
   });
 }
 

@@ -18,6 +18,8 @@ struct mk_ctx {
   char name[64] = {0};
   void* scratch = nullptr;  // per-context device scratch (partial reductions), allocated once at init
   size_t scratch_bytes = 0;
+  void* topk_cand = nullptr;  // topk_workspace() bytes for mk_topk, allocated at init and never moved: a captured graph keeps
+                              // its address
   int32_t* meta = nullptr;  // 64 bytes of per-call metadata (words 0..3: mk_attend_gqa's token layout, 4: attention's
                             // route), allocated at init
 };

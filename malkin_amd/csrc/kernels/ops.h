@@ -229,11 +229,12 @@ void argmax_top2(hipStream_t s, const float* logits, int rows, int n_vocab, int3
 // Stochastic sampling's candidate selection (sampler.cpp:24-36). Row r of a launch is logits row rows[r] (rows null:
 // row r) of `stride` floats. penalize: l[pen_id[i]] -= pen_amt[i] for i in pen_off[r] .. pen_off[r + 1] (ids outside
 // the vocabulary skipped). topk: the k (1..1024) largest logits of each row, highest first, ties by lower id, into
-// values / ids [n_rows][k] (scratch: at least 256 KB, the slices' candidates of rows past 8192 logits).
+// values / ids [n_rows][k] (cand: topk_workspace() bytes, the slices' candidates of rows past 8192 logits).
+size_t topk_workspace();
 void penalize(hipStream_t s, float* logits, int64_t stride, const int32_t* rows, int n_rows, int n_vocab,
               const int32_t* pen_off, const int32_t* pen_id, const float* pen_amt);
 void topk(hipStream_t s, const float* logits, int64_t stride, const int32_t* rows, int n_rows, int n_vocab, int k,
-          float* values, int32_t* ids, void* scratch, size_t scratch_bytes);
+          float* values, int32_t* ids, void* cand);
 size_t sample_cut_workspace(int n_rows, int n_vocab);
 void sample_cut(hipStream_t s, const float* logits, int64_t stride, const int32_t* rows, int n_rows, int n_vocab,
                 const mk_cut_params* params, int cap, float* values, int32_t* ids, int32_t* keep, double* sums,

@@ -7,7 +7,7 @@
 // Top-k per row: the logits become order-preserving 32-bit keys, and a workgroup selects the first of the keys that its
 // threads hold in registers (select_k: a search for the k-th largest key, two bits per step, counted by wave ballots).
 // A long row is cut into kSlices slices of every kSlices-th 64-logit chunk, one workgroup each (k_topk_part); each
-// gives its slice_keep(k) first candidates through the context's scratch, and one workgroup per row selects from those
+// gives its slice_keep(k) first candidates through the context's workspace, and one workgroup per row selects from those
 // and sorts (k_topk_final). Neighbouring ids fall into different slices, so a slice holds about k / kSlices of the
 // row's first k; where all the candidates of a slice were selected, it may hold more, and the row is then walked
 // whole, in rounds of as many logits as the threads hold.
@@ -31,6 +31,9 @@ constexpr int kOneSlice = kFinalPer * kSelThreads;  // logits of a row that one 
 // Candidates that a slice gives: four times the k / kSlices it holds on average, and 16.
 __host__ __device__ constexpr int slice_keep(int k) { return k < 16 + k / 16 ? k : 16 + k / 16; }
 static_assert(kSlices * slice_keep(kMaxTopK) <= kFinalPer * kSelThreads, "one workgroup holds a row's candidates");
+
+// Rows whose candidates the workspace holds, at any k (10 MB).
+constexpr int kSliceRows = 256;
 
 // Logits of a slice, some of them past the row's end.
 __host__ __device__ constexpr int slice_logits(int n_vocab) {
@@ -287,6 +290,8 @@ __global__ __launch_bounds__(kSelThreads) void k_topk_final(const float* __restr
 
 }  // namespace
 
+size_t topk_workspace() { return (size_t)kSliceRows * kSlices * slice_keep(kMaxTopK) * sizeof(uint2); }
+
 void penalize(hipStream_t s, float* logits, int64_t stride, const int32_t* rows, int n_rows, int n_vocab,
               const int32_t* pen_off, const int32_t* pen_id, const float* pen_amt) {
   if (n_rows <= 0) return;
@@ -297,20 +302,19 @@ void penalize(hipStream_t s, float* logits, int64_t stride, const int32_t* rows,
 }
 
 // Rows of up to kOneSlice logits take one workgroup each; longer ones kSlices slices, whose candidates go through the
-// scratch, as many rows per pair of launches as it holds (40 KB per row at k = 1024). Measured, with one
+// workspace, as many rows per pair of launches as it holds. Measured, with one
 // workgroup walking each row -> this form: 8 rows of 151936 at k = 40 276 -> 23 us (1024: 287 -> 48), one row
 // 238 -> 18, 64 rows 407 -> 72, 8 rows of 8193 56 -> 14; of 8192, which one workgroup selects from registers in one
 // round (slices would cost the second launch), 57 -> 17 before the searches ended early. A slice's threads hold 4, 8, 12
 // or 16 logits each, as many as it needs: the searches' ballots are what k_topk_part spends its time on.
 void topk(hipStream_t s, const float* logits, int64_t stride, const int32_t* rows, int n_rows, int n_vocab, int k,
-          float* out_v, int32_t* out_i, void* scratch, size_t scratch_bytes) {
+          float* out_v, int32_t* out_i, void* workspace) {
   if (n_rows <= 0) return;
   require(k >= 1 && k <= kMaxTopK && k <= n_vocab, "topk: k must be 1..1024 and at most the vocabulary");
   const bool sliced = n_vocab > kOneSlice;
   const int keep = slice_keep(k);
-  const int batch = sliced ? (int)std::min<size_t>(n_rows, scratch_bytes / (kSlices * keep * sizeof(uint2))) : n_rows;
-  require(batch > 0, "topk: scratch too small");
-  uint2* cand = sliced ? static_cast<uint2*>(scratch) : nullptr;
+  const int batch = sliced ? std::min(n_rows, kSliceRows) : n_rows;
+  uint2* cand = sliced ? static_cast<uint2*>(workspace) : nullptr;
   for (int r0 = 0; r0 < n_rows; r0 += batch) {
     const int nr = std::min(batch, n_rows - r0);
     const float* l = rows ? logits : logits + (int64_t)r0 * stride;
