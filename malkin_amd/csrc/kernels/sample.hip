@@ -6,7 +6,7 @@
 //
 // Top-k per row: the logits become order-preserving 32-bit keys, and a workgroup selects the first of the keys that its
 // threads hold in registers (select_k: a search for the k-th largest key, two bits per step, counted by wave ballots).
-// A long row is cut into kSlices slices of every kSlices-th 64-logit chunk, one workgroup each (k_topk_part); each
+// A long row of few is cut into kSlices slices of every kSlices-th 64-logit chunk, one workgroup each (k_topk_part); each
 // gives its slice_keep(k) first candidates through the context's workspace, and one workgroup per row selects from those
 // and sorts (k_topk_final). Neighbouring ids fall into different slices, so a slice holds about k / kSlices of the
 // row's first k; where all the candidates of a slice were selected, it may hold more, and the row is then walked
@@ -32,7 +32,7 @@ constexpr int kOneSlice = kFinalPer * kSelThreads;  // logits of a row that one 
 __host__ __device__ constexpr int slice_keep(int k) { return k < 16 + k / 16 ? k : 16 + k / 16; }
 static_assert(kSlices * slice_keep(kMaxTopK) <= kFinalPer * kSelThreads, "one workgroup holds a row's candidates");
 
-// Rows whose candidates the workspace holds, at any k (10 MB).
+// Rows that are selected from in slices at most: the workspace holds their candidates at any k (10 MB).
 constexpr int kSliceRows = 256;
 
 // Logits of a slice, some of them past the row's end.
@@ -176,8 +176,11 @@ __global__ __launch_bounds__(kPartThreads) void k_topk_part(const float* __restr
 }
 
 // One row's k first, sorted: from its slices' candidates (cand[row][kSlices][keep]), or from the row itself (cand NULL;
-// also where a slice's candidates were all selected), in rounds of the keys the threads hold and the best so far.
-__global__ __launch_bounds__(kSelThreads) void k_topk_final(const float* __restrict__ logits, int64_t stride,
+// also where a slice's candidates were all selected), in rounds of the keys the threads hold and the best so far. WAVES: per
+// SIMD; 8 put two rows on a CU (512 rows of 151936 at k = 40 404 -> 294 us) but have the searches' counts spill to lanes of
+// vector registers, which costs a walked row that has its CU alone 3 %.
+template <int WAVES>
+__global__ __launch_bounds__(kSelThreads) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_topk_final(const float* __restrict__ logits, int64_t stride,
                                                              const int32_t* __restrict__ rows, int n_vocab,
                                                              const uint2* __restrict__ cand, int k,
                                                              float* __restrict__ out_v, int32_t* __restrict__ out_i) {
@@ -301,37 +304,35 @@ void penalize(hipStream_t s, float* logits, int64_t stride, const int32_t* rows,
   check_launch("penalize");
 }
 
-// Rows of up to kOneSlice logits take one workgroup each; longer ones kSlices slices, whose candidates go through the
-// workspace, as many rows per pair of launches as it holds. Measured, with one
-// workgroup walking each row -> this form: 8 rows of 151936 at k = 40 276 -> 23 us (1024: 287 -> 48), one row
-// 238 -> 18, 64 rows 407 -> 72, 8 rows of 8193 56 -> 14; of 8192, which one workgroup selects from registers in one
-// round (slices would cost the second launch), 57 -> 17 before the searches ended early. A slice's threads hold 4, 8, 12
+// Rows of up to kOneSlice logits take one workgroup each, and so do longer rows where there are many of them: slices pay
+// while the chip would be idle, but cost a row 64 workgroups of its own. A row of n logits walked by one workgroup takes
+// about as long as slices of n / 256 rows (us, walked / slices: 64 rows of 8193 at k = 40 17 / 26, 8 rows 16 / 15; 128 rows of
+// 32768 51 / 42, 256 rows 51 / 70; 256 rows of 151936 209 / 228, 64 rows 209 / 68). Past kSliceRows rows the walks fill the
+// chip. Against one workgroup walking each row by histograms (this file's first form): 8 rows of 151936 at k = 40
+// 276 -> 21 us (1024: 287 -> 46), one row 238 -> 18, 64 rows 387 -> 68, 512 rows 461 -> 294; 8 rows of 8193 56 -> 15, 256 rows
+// 59 -> 17, and of 8192, which one workgroup selects from registers in one round, 57 -> 12. A slice's threads hold 4, 8, 12
 // or 16 logits each, as many as it needs: the searches' ballots are what k_topk_part spends its time on.
 void topk(hipStream_t s, const float* logits, int64_t stride, const int32_t* rows, int n_rows, int n_vocab, int k,
           float* out_v, int32_t* out_i, void* workspace) {
   if (n_rows <= 0) return;
   require(k >= 1 && k <= kMaxTopK && k <= n_vocab, "topk: k must be 1..1024 and at most the vocabulary");
-  const bool sliced = n_vocab > kOneSlice;
-  const int keep = slice_keep(k);
-  const int batch = sliced ? std::min(n_rows, kSliceRows) : n_rows;
+  const bool sliced = n_vocab > kOneSlice && n_rows <= std::min(n_vocab / 256, kSliceRows);
   uint2* cand = sliced ? static_cast<uint2*>(workspace) : nullptr;
-  for (int r0 = 0; r0 < n_rows; r0 += batch) {
-    const int nr = std::min(batch, n_rows - r0);
-    const float* l = rows ? logits : logits + (int64_t)r0 * stride;
-    const int32_t* rr = rows ? rows + r0 : nullptr;
+  if (sliced) {
     auto part = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(kSlices, nr), dim3(kPartThreads), 0, s, l, stride, rr, n_vocab, keep, cand);
+      hipLaunchKernelGGL(kernel, dim3(kSlices, n_rows), dim3(kPartThreads), 0, s, logits, stride, rows, n_vocab,
+                         slice_keep(k), cand);
     };
-    if (sliced) {
-      const int per = (slice_logits(n_vocab) + kPartThreads - 1) / kPartThreads;
-      per <= 4    ? part(k_topk_part<4>)
-      : per <= 8  ? part(k_topk_part<8>)
-      : per <= 12 ? part(k_topk_part<12>)
-                  : part(k_topk_part<16>);
-    }
-    hipLaunchKernelGGL(k_topk_final, dim3(nr), dim3(kSelThreads), 0, s, l, stride, rr, n_vocab, cand, k,
-                       out_v + (int64_t)r0 * k, out_i + (int64_t)r0 * k);
+    const int per = (slice_logits(n_vocab) + kPartThreads - 1) / kPartThreads;
+    per <= 4    ? part(k_topk_part<4>)
+    : per <= 8  ? part(k_topk_part<8>)
+    : per <= 12 ? part(k_topk_part<12>)
+                : part(k_topk_part<16>);
   }
+  auto final = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(n_rows), dim3(kSelThreads), 0, s, logits, stride, rows, n_vocab, cand, k, out_v, out_i);
+  };
+  n_rows > device_cus() ? final(k_topk_final<8>) : final(k_topk_final<4>);
   check_launch("topk");
 }
 

@@ -1,4 +1,5 @@
-"""mk_topk in a captured graph, which keeps selecting right when the context's scratch has moved since the capture."""
+"""mk_topk in a captured graph, which keeps selecting right when the context's scratch has moved since the capture, and over
+many rows, which are walked by one workgroup each instead of cut into slices."""
 import ctypes
 
 import numpy as np
@@ -44,3 +45,20 @@ def test_graph_outlives_scratch():
     for b in others + [dx, dv, di]:
         b.free()
     ctx.close()
+
+
+@pytest.mark.parametrize("V,k,n_rows", [(8193, 1, 70000), (8193, 1024, 32), (8193, 1024, 33), (9000, 40, 300),
+                                        (65792, 1024, 256), (65792, 1024, 257), (1 << 18, 300, 257)])
+def test_many_rows(mk, V, k, n_rows):
+    """n_rows rows that are five logits rows over and over, around the count from which one workgroup walks a row."""
+    rng = np.random.default_rng(V)
+    x = rng.standard_normal((5, V)).astype(np.float32)
+    rows = (np.arange(n_rows) * 3 % 5).astype(np.int32)
+    dx, dr = mk.to_device(x), mk.to_device(rows)
+    dv, di = mk.alloc(n_rows * k * 4), mk.alloc(n_rows * k * 4)
+    print("topk many rows", V, k, n_rows, flush=True)
+    mk_.check(mk_.load().mk_topk(mk.h, dx.ptr, V, dr.ptr, n_rows, V, k, dv.ptr, di.ptr))
+    gv, gi = dv.download(np.uint32).reshape(n_rows, k), di.download(np.int32).reshape(n_rows, k)
+    for r in range(5):
+        ev, ei = expected_topk(x[r], k)
+        assert (gi[rows == r] == ei).all() and (gv[rows == r] == ev.view(np.uint32)).all()
