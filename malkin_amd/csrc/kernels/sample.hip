@@ -9,11 +9,13 @@
 // A long row of few is cut into kSlices slices of every kSlices-th 64-logit chunk, one workgroup each (k_topk_part); each
 // gives its slice_keep(k) first candidates through the context's workspace, and one workgroup per row selects from those
 // and sorts (k_topk_final). Neighbouring ids fall into different slices, so a slice holds about k / kSlices of the
-// row's first k; where all the candidates of a slice were selected, it may hold more, and the row is then walked
-// whole, in rounds of as many logits as the threads hold.
+// row's first k; where all the candidates of a slice were selected, it may hold more, and that slice is then walked
+// whole, in rounds of as many logits as the threads hold (the whole row: one row of 151936 whose first 1024 fall into one
+// slice 282 us, that slice 55).
 // What bounds it: two launches and the searches' barriers; the logits are read once (4.9 MB for 8 rows of 151936). See
 // topk() for the times.
 #include <algorithm>
+#include <type_traits>
 
 #include "ctx.h"
 #include "ops.h"
@@ -93,9 +95,9 @@ struct SelLds {
   uint32_t gt, eq, slot;
 };
 
-// put(slot, key, id) for the k first keys of the workgroup in the order (key desc, id asc), slots in any order. Threads
-// without a key hold (0, INT32_MAX), below every logit's key; where fewer than k hold one, T is 0, every key is put and
-// some slots are k or more (put drops those, and keys of 0 come last in no order: see below).
+// put(slot, key, id) for the k first keys of the workgroup in the order (key desc, id asc), slots 0 .. k - 1 in any order;
+// returns how many. Threads without a key hold (0, INT32_MAX), below every logit's key; where fewer than k hold one, T is 0
+// and only the keys above 0 are put.
 template <int E, class Put>
 __device__ __forceinline__ int select_k(const uint32_t (&key)[E], const int32_t (&id)[E], int k, SelLds& L, Put put) {
   const int tid = threadIdx.x, lane = tid & 63;
@@ -175,28 +177,27 @@ __global__ __launch_bounds__(kPartThreads) void k_topk_part(const float* __restr
   }
 }
 
-// One row's k first, sorted: from its slices' candidates (cand[row][kSlices][keep]), or from the row itself (cand NULL;
-// also where a slice's candidates were all selected), in rounds of the keys the threads hold and the best so far. WAVES: per
-// SIMD; 8 put two rows on a CU (512 rows of 151936 at k = 40 404 -> 294 us) but have the searches' counts spill to lanes of
-// vector registers, which costs a walked row that has its CU alone 3 %.
-template <int WAVES>
-__global__ __launch_bounds__(kSelThreads) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_topk_final(const float* __restrict__ logits, int64_t stride,
-                                                             const int32_t* __restrict__ rows, int n_vocab,
-                                                             const uint2* __restrict__ cand, int k,
-                                                             float* __restrict__ out_v, int32_t* __restrict__ out_i) {
+// One row's k first, sorted: from its slices' candidates (SLICED: cand[row][kSlices][keep]) and the logits of those slices
+// whose candidates were all selected, or from the row's logits, in rounds of the keys the threads hold and the best so
+// far. WAVES: per SIMD; 8 put two rows on a CU (512 rows of 151936 at k = 40 404 -> 294 us) but have the searches' counts
+// spill to lanes of vector registers, which costs a walked row that has its CU alone 3 %.
+template <int WAVES, bool SLICED>
+__global__ __launch_bounds__(kSelThreads) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_topk_final(
+    const float* __restrict__ logits, int64_t stride, const int32_t* __restrict__ rows, int n_vocab,
+    const uint2* __restrict__ cand, int k, float* __restrict__ out_v, int32_t* __restrict__ out_i) {
   constexpr int E = kFinalPer, NT = kSelThreads;
   __shared__ SelLds L;
   __shared__ uint32_t ckey[kMaxTopK];
   __shared__ int32_t cidx[kMaxTopK];
-  __shared__ int taken[kSlices], again;
+  __shared__ int taken[kSlices], full[kSlices], n_full, again;
   const int tid = threadIdx.x, r = blockIdx.x;
   const int keep = slice_keep(k);
+  auto slice_of = [](int32_t i) { return (int)((uint32_t)i / kChunk % kSlices); };
   auto put = [&](uint32_t slot, uint32_t kk, int32_t ii) {
     ckey[slot] = kk;
     cidx[slot] = ii;
   };
-  bool walk = cand == nullptr;
-  if (!walk) {
+  if constexpr (SLICED) {
     const int n = kSlices * keep;
     const uint2* c = cand + (int64_t)r * n;
     if (tid < kSlices) taken[tid] = 0;
@@ -219,22 +220,44 @@ __global__ __launch_bounds__(kSelThreads) __attribute__((amdgpu_waves_per_eu(WAV
       from_cand.template operator()<E>();
     __syncthreads();
     for (int i = tid; i < k; i += NT)
-      if (atomicAdd(&taken[(uint32_t)cidx[i] / kChunk % kSlices], 1) + 1 >= keep && keep < k) again = 1;
+      if (atomicAdd(&taken[slice_of(cidx[i])], 1) + 1 >= keep && keep < k) again = 1;
     __syncthreads();
-    walk = again != 0;
+    if (again) {
+      if (tid < kSlices) {
+        const unsigned long long bal = __ballot(taken[tid] >= keep);
+        if (taken[tid] >= keep) full[__popcll(bal & ((1ull << tid) - 1ull))] = tid;
+        if (tid == 0) n_full = __popcll(bal);
+      }
+      // The walk meets these slices' candidates again. (Entry i is read there by the thread that clears it.)
+      for (int i = tid; i < k; i += NT)
+        if (taken[slice_of(cidx[i])] >= keep) put(i, 0u, INT32_MAX);
+      __syncthreads();
+    }
   }
+  // The row's logits, or those of its full slices.
+  using Pos = std::conditional_t<SLICED, int64_t, int>;
+  const uint32_t nsl = (uint32_t)slice_logits(n_vocab);
+  const Pos walk = !SLICED ? (Pos)n_vocab : again ? (Pos)n_full * nsl : 0;
   if (walk) {
     const float* l = logits + (int64_t)(rows ? rows[r] : r) * stride;
     uint32_t key[E];
     int32_t id[E];
-    for (int pos = 0, held = 0; pos < n_vocab;) {
-      const int take = min(n_vocab - pos, E * NT - held);
+    int held = SLICED ? k : 0;
+    for (Pos pos = 0; pos < walk;) {
+      const int take = (int)min(walk - pos, (Pos)(E * NT - held));
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const int i = e * NT + tid, j = i - held;
-        const bool in = j >= 0 && j < take;
-        id[e] = in ? pos + j : i < held ? cidx[i] : INT32_MAX;
-        key[e] = in ? order_key(l[pos + j]) : i < held ? ckey[i] : 0u;
+        bool in = j >= 0 && j < take;
+        Pos v = pos + j;
+        if constexpr (SLICED)
+          if (in) {
+            const uint32_t q = (uint32_t)v, c = q % nsl;
+            v = ((Pos)(c / kChunk) * kSlices + full[q / nsl]) * kChunk + c % kChunk;
+            in = v < n_vocab;
+          }
+        id[e] = in ? (int32_t)v : i < held ? cidx[i] : INT32_MAX;
+        key[e] = in ? order_key(l[v]) : i < held ? ckey[i] : 0u;
       }
       __syncthreads();  // the best so far have been read
       select_k(key, id, k, L, put);
@@ -332,7 +355,9 @@ void topk(hipStream_t s, const float* logits, int64_t stride, const int32_t* row
   auto final = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(n_rows), dim3(kSelThreads), 0, s, logits, stride, rows, n_vocab, cand, k, out_v, out_i);
   };
-  n_rows > device_cus() ? final(k_topk_final<8>) : final(k_topk_final<4>);
+  sliced                  ? final(k_topk_final<4, true>)
+  : n_rows > device_cus() ? final(k_topk_final<8, false>)
+                          : final(k_topk_final<4, false>);
   check_launch("topk");
 }
 

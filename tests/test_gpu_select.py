@@ -35,3 +35,21 @@ def test_topk_forms(mk, V, k, n_rows):
         ev, ei = expected_topk(x[r], k)
         assert np.array_equal(gi[r], ei), (V, k, r)
         assert np.array_equal(gv[r].view(np.uint32), ev.view(np.uint32)), (V, k, r)
+
+
+@pytest.mark.parametrize("V,k", [(8193, 40), (8193, 1024), (20000, 256), (151936, 18), (151936, 1024), (1 << 19, 700)])
+@pytest.mark.parametrize("n_full", [1, 3, 64])
+def test_topk_full_slices(mk, V, k, n_full):
+    """Rows whose largest logits fall into n_full of the 64 slices, with ties, distinct or all equal."""
+    rng = np.random.default_rng(V + k + n_full)
+    x = rng.standard_normal((3, V)).astype(np.float32)
+    x[:, np.isin(np.arange(V) // 64 % 64, rng.permutation(64)[:n_full])] += 8.0
+    x[1] = np.round(x[1])
+    x[2] = 0.5
+    dx, dv, di = mk.to_device(x), mk.alloc(3 * k * 4), mk.alloc(3 * k * 4)
+    print("topk full slices", V, k, n_full, flush=True)
+    mk_.check(mk_.load().mk_topk(mk.h, dx.ptr, V, None, 3, V, k, dv.ptr, di.ptr))
+    gv, gi = dv.download(np.uint32).reshape(3, k), di.download(np.int32).reshape(3, k)
+    for r in range(3):
+        ev, ei = expected_topk(x[r], k)
+        assert np.array_equal(gi[r], ei) and np.array_equal(gv[r], ev.view(np.uint32)), (V, k, n_full, r)
