@@ -8,6 +8,7 @@
 //   bias chains).
 // A wave holds four groups, a workgroup sixteen: one weight row per group, NT tokens of it at once so that a row is read
 // once per token tile. F32 / F16 / BF16 rows go to the matrix cores instead (k_rows_mfma) unless they are unaligned.
+#include <algorithm>
 #include <utility>
 
 #include "ctx.h"
@@ -634,6 +635,13 @@ void matmul_rows(hipStream_t s, int type, const void* w, size_t row_bytes, int64
   const bool f = type == kF32 || type == kF16 || type == kBF16;
   require(f ? x != nullptr : xq != nullptr, "matmul_rows: missing activations (fp32 for F32/F16/BF16, BlockQ8 else)");
   if (rows_mfma_ok(type, w, row_bytes, rows, cols, x, xs, n)) {
+    // A launch has less than 2^32 threads, 2^24 workgroups here; a batch that large runs in 32 x 32 tiles.
+    const int64_t most = ((int64_t)1 << 24) - 1, row_tiles = (rows + 31) / 32, per = 32 * std::max<int64_t>(1, most / row_tiles);
+    if (n > per) {
+      matmul_rows(s, type, w, row_bytes, rows, cols, x, xs, xq, (int)per, y, ys, accumulate);
+      matmul_rows(s, type, w, row_bytes, rows, cols, x + per * xs, xs, xq, n - (int)per, y + per * ys, ys, accumulate);
+      return;
+    }
     auto* wb = static_cast<const uint8_t*>(w);
     if (type == kF32)
       launch_rows_mfma<kF32>(s, wb, row_bytes, rows, cols, x, xs, n, y, ys, accumulate);
@@ -667,6 +675,11 @@ void matmul_gguf(hipStream_t s, int type, const void* w, size_t row_bytes, int64
           "matmul_gguf: Q4_K / Q5_K rows of a multiple of 256 values");
   require(xq != nullptr, "matmul_gguf: missing activations");
   if (rows <= 0 || n <= 0) return;
+  if (const int most = 1 << 17; n > most) {  // a grid has at most 65536 groups of tokens
+    matmul_gguf(s, type, w, row_bytes, rows, cols, xq, most, y, ys, accumulate);
+    matmul_gguf(s, type, w, row_bytes, rows, cols, xq + most * (cols / 32), n - most, y + most * ys, ys, accumulate);
+    return;
+  }
   if (row_bytes % 16 == 0 && (uintptr_t)w % 16 == 0) {
     // Q5_K batches: the GEMV's waves (4 rows each, a group of 4 tokens) cost about 0.85 us per pass of 512 columns and
     // wave of a SIMD, the MFMA kernel about 3.1 us per 512 columns whatever the batch (up to 32 tokens), so it takes

@@ -165,3 +165,33 @@ def test_q5k_model_golden(mk, model_files, golden):
         assert np.array_equal(bits(m.forward_batch(batch)), bits(g[f"{name}_tree_logits"]))
     finally:
         m.close()
+
+
+def test_gguf_more_tokens_than_a_grid(mk, oracle):
+    """A batch whose groups of four tokens are more than a grid's second dimension holds."""
+    import make_golden
+    rng = np.random.default_rng(17)
+    rows, k, n, few = 3, 256, 262144 + 9, 64
+    w = make_golden.random_rows(rng, bind.Q4_K, rows, k)
+    xq = oracle.quantize_row_q8(rng.uniform(-2, 2, (few, k)).astype(np.float32))
+    exp = oracle.matmul(bind.Q4_K, w, rows, k, xq.reshape(-1))
+    pick = (np.arange(n) * 5 % few).astype(np.int32)
+    blocks = np.ascontiguousarray(xq).view(np.uint8).reshape(few, -1)
+    dw, dq, dy = mk.to_device(w), mk.to_device(blocks[pick]), mk.alloc(n * rows * 4)
+    print("gguf", n, "tokens", flush=True)
+    mk_.check(mk_.load().mk_matmul_gguf(mk.h, bind.Q4_K, dw.ptr, w.shape[1], rows, k, dq.ptr, n, dy.ptr, rows, 0))
+    assert np.array_equal(bits(dy.download(np.float32).reshape(n, rows)), bits(exp[pick]))
+
+
+def test_rows_more_tiles_than_a_grid(mk, oracle):
+    """2^24 tiles of 32 x 32 outputs. Every token reads one row of x and writes one row of y, which keeps both small."""
+    rng = np.random.default_rng(18)
+    rows, k, n, few = 1 << 22, 16, 4100, 256
+    w = (rng.standard_normal((few, k)) * 0.1).astype(np.float16)
+    x = rng.uniform(-2, 2, (1, k)).astype(np.float32)
+    exp = oracle.matmul_rows(bind.F16, w.view(np.uint8).reshape(few, -1), few, k, x=x, xq=None, n=1)
+    dw = mk.to_device(np.tile(w, (rows // few, 1)))
+    dx, dy = mk.to_device(x), mk.alloc(rows * 4)
+    print("rows", rows, "x", n, "tokens", flush=True)
+    mk_.check(mk_.load().mk_matmul_rows(mk.h, bind.F16, dw.ptr, 2 * k, rows, k, dx.ptr, 0, None, n, dy.ptr, 0, 0))
+    assert np.array_equal(bits(dy.download(np.float32).reshape(-1, few)), bits(np.tile(exp, (rows // few, 1))))
