@@ -23,6 +23,9 @@ CASES = [  # H, KV, tokens, tokens of sequence 1, tokens of each other one, long
     (8, 8, 130, 130, 1, 1900),   # matrix cores: one sequence, of a cache of several
     (8, 8, 130, 90, 1, 1900),    # grouped
     (32, 8, 70, 70, 1, 2000),    # matrix cores
+    (24, 8, 73, 73, 1, 1900),    # matrix cores, blocks of 5 tokens
+    (40, 8, 71, 71, 1, 1990),    # matrix cores, blocks of 3 tokens
+    (16, 1, 520, 520, 1, 1870),  # matrix cores, blocks of one token
     (32, 8, 70, 33, 1, 2000),    # grouped
     (32, 8, 67, 0, 2, 3000),     # matrix cores, two sequences a block
     (32, 8, 70, 33, 1, 3000),    # grouped, a group's heads in workgroups of their own

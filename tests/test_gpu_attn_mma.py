@@ -1,6 +1,7 @@
 """Prompt-chunk attention on the fp32 matrix cores (head_dim 128, 16 tokens or more), bit for bit against the oracle's
 attend_gqa: keys around its 16-key tiles and 64-key stages, G that does not divide 16, blocks of mixed sequences, the
-longest rows its LDS holds (1856 keys), and longer ones in 512-key chunks."""
+longest rows its LDS holds (1856 keys), and just longer ones, which its form of 512-key chunks or the grouped kernel takes
+(test_gpu_attn_mixed.py has that form's cases)."""
 import ctypes
 
 import numpy as np

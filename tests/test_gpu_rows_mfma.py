@@ -1,7 +1,7 @@
 """mk_matmul_rows for F32 / F16 / BF16 rows on the matrix cores, bit for bit against the CPU oracle, where the kernel's
-forms and edges meet: few tokens (4 staged) and one workgroup per CU, 16 x 16, 16 x 32 and 32 x 32 tiles, rows and
-tokens past the last tile, partial 64-column steps, k % 16 tails, strided activations, and the unaligned rows
-that keep the lane-group kernel. Weights and activations hold signed zeros and denormals."""
+forms and edges meet: few tokens (4 staged) on one and several workgroups per CU, 16 x 16, 16 x 32 and 32 x 32 tiles, each
+over more stages than its ring holds, rows and tokens past the last tile, partial 64-column steps, k % 16 tails,
+strided activations, and the unaligned rows that keep the lane-group kernel. Weights and activations hold signed zeros and denormals."""
 import numpy as np
 import pytest
 
@@ -12,7 +12,9 @@ from test_gpu_rowpath import bits, row_weights
 pytestmark = pytest.mark.gpu
 
 CASES = [(40, 16, 1), (40, 4100, 4), (4104, 80, 4), (4104, 80, 5), (24, 1032, 16), (56, 200, 33), (4000, 72, 50),
-         (8200, 144, 97), (8193, 64, 128), (24, 36, 3), (24, 100, 20)]
+         (8200, 144, 97), (8193, 64, 128), (24, 36, 3), (24, 100, 20),
+         # on 256 CUs the 4-token form past one tile per CU, 16 x 32 and 32 x 32 tiles, over 5 or 6 stages of their rings
+         (4104, 1300, 4), (4000, 520, 50), (8200, 652, 97)]
 
 
 @pytest.mark.parametrize("t", [bind.F32, bind.F16, bind.BF16])
