@@ -70,8 +70,8 @@ struct TokenLayout {
   // Tree batches: token t attends to its n_keys[t] contiguous rows, then to rows extra[extra_at[t] .. extra_at[t+1]).
   bool tree = false;
   std::vector<int32_t> extra_at, extra;
-  // Derived: the longest key list, whether no two tokens share a sequence, and what a plain batch's attention on the matrix
-  // cores would walk.
+  // Derived: the longest key list, whether no two tokens share a sequence, and what a plain batch's attention on the
+  // matrix cores would walk.
   int max_keys = 0;
   bool distinct_seqs = false;
   mk::AttnWalks walks;

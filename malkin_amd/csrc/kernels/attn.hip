@@ -912,20 +912,21 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention_grp(const float* __r
   }
 }
 
-// Whether attention_mma takes a plain batch of rows longer than its LDS holds: its walks, in rounds of the CUs (one workgroup
-// per KV head and token block, one walk after the other), cost no more than `rest`, the kernel that takes the tokens
-// otherwise (rest_cost). Units of 1/200 of a walk. Where about every block has as many walks as the longest, a round lasts
-// that long; a few long blocks fill the others' rounds in part.
+// Whether attention_mma takes a plain batch of rows longer than its LDS holds: its walks, in rounds of the CUs (one
+// workgroup per KV head and token block, one walk after the other), cost no more than `rest`, the kernel that takes the
+// tokens otherwise (rest_cost). Units of 1/200 of a walk. Where about every block has as many walks as the longest, a
+// round lasts that long; a few long blocks fill the others' rounds in part.
 __host__ __device__ inline bool mma_pays(const AttnWalks& w, int blocks, int KV, int cus, int rest) {
   auto rounds = [&](int64_t n) { return (int)((n * KV + cus - 1) / cus); };
   const int even = rounds(w.all), full = min(even + w.most - 1, rounds(blocks) * w.most);
-  const int r = 4 * (int64_t)w.all >= 3 * (int64_t)blocks * w.most ? full : min(full, max(even, w.most) + (w.most - 1) / 2);
+  const bool alike = 4 * (int64_t)w.all >= 3 * (int64_t)blocks * w.most;
+  const int r = alike ? full : min(full, max(even, w.most) + (w.most - 1) / 2);
   return 200 * (int64_t)r <= rest;
 }
 
 // Whether a plain batch's walks pay, for callers whose sequences only the device knows. 16 lanes per token block.
-__global__ __launch_bounds__(1024) void k_attention_route(const int32_t* __restrict__ seqs, int n, int TQ, int KV, int cus,
-                                                          int rest, int32_t* __restrict__ route) {
+__global__ __launch_bounds__(1024) void k_attention_route(const int32_t* __restrict__ seqs, int n, int TQ, int KV,
+                                                          int cus, int rest, int32_t* __restrict__ route) {
   __shared__ int all_s, most_s;
   if (threadIdx.x == 0) all_s = most_s = 0;
   __syncthreads();
@@ -1466,9 +1467,10 @@ int grp_heads(int n, int H, int G, int D, const AttnAddr& a, const int32_t* anc_
   return grp_lds_bytes(1, nk_pad, anc_cap) <= limit ? 1 : 0;
 }
 
-// What the batch costs without attention_mma, in 1/200 of a walk of its workgroups over the keys: rounds of the grouped kernel
-// (GH heads a workgroup; 52, 65, 72 and 97 us at 1, 2, 4 and 5 heads where a walk takes 177, at 4000 keys; the same shares
-// from 2000 to 8000), past that one's keys of k_attention_long (as much as a walk).
+// What the batch costs without attention_mma, in 1/200 of a walk of its workgroups over the keys: rounds of the grouped
+// kernel (GH heads a workgroup: 53 and 65 us at 1 and 2 heads over 4000 keys, where a walk takes 177; 43, 42 and 51 at 3, 4
+// and 5 over 2000, where it takes 92; the shares hold from 2000 to 8000 keys), past that one's keys of k_attention_long
+// (360 to 520 over 12000, where a walk takes 519).
 int rest_cost(int n, int KV, int G, int GH) {
   const int64_t cus = device_cus(), wgs = (int64_t)n * KV * (GH > 0 ? (G + GH - 1) / GH : G);
   return (int)std::min<int64_t>(INT32_MAX, (wgs + cus - 1) / cus * (GH > 0 ? 47 + 12 * GH : 190));
@@ -1487,8 +1489,8 @@ void with_heads(int GH, F go) {
 
 void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int64_t out_stride, int n, int H, int KV,
                int D, float scale, const AttnAddr& a, const int32_t* seq, const int32_t* n_keys,
-               const int32_t* anc_off, const int32_t* anc, int max_keys, int n_seq, const AttnWalks* walks, int32_t* route,
-               void* scratch, size_t scratch_bytes, BlockQ8* xq, int64_t xq_stride) {
+               const int32_t* anc_off, const int32_t* anc, int max_keys, int n_seq, const AttnWalks* walks,
+               int32_t* route, void* scratch, size_t scratch_bytes, BlockQ8* xq, int64_t xq_stride) {
   if (n <= 0) return;
   require(D % 16 == 0 && D <= 256 && H % KV == 0 && max_keys > 0, "attention: unsupported head layout");
   require(!xq || D % 32 == 0, "attention: Q8 rows need head_dim % 32 == 0");
@@ -1497,11 +1499,12 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
   const int GH = grp_heads(n, H, G, D, a, anc_off, max_keys);
   // Many plain tokens on the matrix cores: always where a row's scores fit LDS. Longer rows, whose scores run twice, where
   // the batch takes more than two rounds of the CUs otherwise and its walks pay (mma_pays); where only the device knows
-  // the sequences and they matter, it decides: both kernels are launched and one of them leaves at once (4 to 9 us). Measured at
-  // 32 heads over 8 KV heads, the grouped kernel / this, us: 128 tokens of one sequence over 2000 keys 169 / 92, of 64
-  // sequences 171 / 187, of 128 180 / 366; 128 tokens over 3000 keys, where a group's heads take workgroups of their own,
-  // 645 / 133, 534 / 279 and 541 / 500; 8 heads over 8 KV heads, 80 tokens of one sequence over 4000 keys 159 / 177.
-  // (Past the grouped kernel's keys the caller's scratch must hold a row all the same: such calls have always needed it.)
+  // the sequences and they matter, it decides: both kernels are launched and one of them leaves at once (4 to 9 us).
+  // Measured at 32 heads over 8 KV heads, the grouped kernel / this, us: 128 tokens of one sequence over 2000 keys
+  // 169 / 92, of 64 sequences 171 / 187, of 128 180 / 366; 128 tokens over 6000 keys, where a group's heads take workgroups
+  // of their own, 1229 / 262, 1233 / 554 and 1238 / 1083; 8 heads over 8 KV heads, 80 tokens of one sequence over 4000 keys
+  // 159 / 177. (Past the grouped kernel's keys the caller's scratch must hold a row all the same: such calls have always
+  // needed it.)
   const int32_t* routed = nullptr;
   if (!anc_off && n >= kRowsMinTokens && attention_mma_ok(G, D, a)) {
     bool mma = attention_mma_whole(max_keys);

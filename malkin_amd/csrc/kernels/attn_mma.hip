@@ -22,7 +22,7 @@
 //
 // What bounds it: fp32 MFMAs and vector instructions share a SIMD's issue (measured: they do not overlap), so a 16-key
 // score tile costs 32 x 32 cycles of MFMA and about 150 vector instructions (transpose, conversions, the trees), and
-// P.V 32 cycles per 4 keys and wave. 512 tokens of 32 heads over 8 KV heads (16-row workgroups, one per CU past 850
+// P.V 32 cycles per 4 keys and wave. 512 tokens of 32 heads over 8 KV heads (16-row workgroups, one per CU past 704
 // keys), us against the vector kernel this replaced (one key per thread, fp32 V tiles): first chunk 81 -> 58, behind 512
 // tokens 320 -> 122, behind 1024 506 -> 184. With one scalar byte read of V per value instead of the transposing LDS
 // read, and the K loads left to the compiler's order (behind half of the tile's MFMAs): 134 instead of 122.

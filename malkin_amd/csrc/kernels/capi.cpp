@@ -417,7 +417,8 @@ AttnWalks attention_walks(const int32_t* host_seq, int n, int G) {
   const int tq = 16 / std::min(std::max(G, 1), 16);
   for (int t0 = 0; t0 < n; t0 += tq) {
     int c = 0;
-    for (int t = t0; t < std::min(t0 + tq, n); ++t) c += std::find(host_seq + t0, host_seq + t, host_seq[t]) == host_seq + t;
+    for (int t = t0; t < std::min(t0 + tq, n); ++t)
+      if (std::find(host_seq + t0, host_seq + t, host_seq[t]) == host_seq + t) ++c;
     w.all += c;
     w.most = std::max(w.most, c);
   }
@@ -428,7 +429,8 @@ int attention_batch(mk_ctx* c, const float* q, int64_t q_stride, float* out, int
                     const mk_kv_cache* kv, int layer, const int32_t* seq, const int32_t* n_keys, const int32_t* anc_off,
                     const int32_t* anc, int max_keys, void* xq, const AttnWalks* walks) {
   return guard([&] {
-    attention_rows(c, q, q_stride, out, out_stride, n, n_head, kv, layer, seq, n_keys, anc_off, anc, max_keys, xq, walks);
+    attention_rows(c, q, q_stride, out, out_stride, n, n_head, kv, layer, seq, n_keys, anc_off, anc, max_keys, xq,
+                   walks);
   });
 }
 }  // namespace mk

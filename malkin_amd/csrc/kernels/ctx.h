@@ -66,8 +66,8 @@ void allow_lds(int bytes) {
   (void)set;
 }
 
-// The walks over a sequence's keys that attention on the matrix cores makes for a plain batch, per KV head: for each block
-// of 16 / G consecutive tokens one per sequence among them. All blocks' and the most of one block.
+// The walks over a sequence's keys that attention on the matrix cores makes for a plain batch, per KV head: for each
+// block of 16 / G consecutive tokens one per sequence among them. All blocks' and the most of one block.
 struct AttnWalks {
   int all = 0, most = 0;
 };

@@ -101,22 +101,6 @@ __device__ __forceinline__ v16f conv(v16i c) {
 // q - 32 per byte for bytes q < 64.
 __device__ __forceinline__ uint32_t minus32(uint32_t q) { return ((q | 0x80808080u) - 0x20202020u) ^ 0x80808080u; }
 
-// scale_min_k4 (the reference's kernels.h:18-26) of the 12 packed scale bytes held in q0..q2.
-__device__ __forceinline__ int kbyte(uint32_t q0, uint32_t q1, uint32_t q2, int i) {
-  const uint32_t w = i < 4 ? q0 : (i < 8 ? q1 : q2);
-  return (int)((w >> (8 * (i & 3))) & 0xFFu);
-}
-__device__ __forceinline__ void scale_min(int j, uint32_t q0, uint32_t q1, uint32_t q2, int& sc, int& m) {
-  if (j < 4) {
-    sc = kbyte(q0, q1, q2, j) & 63;
-    m = kbyte(q0, q1, q2, j + 4) & 63;
-  } else {
-    const int hi = kbyte(q0, q1, q2, j + 4);
-    sc = (hi & 0xF) | ((kbyte(q0, q1, q2, j - 4) >> 6) << 4);
-    m = (hi >> 4) | ((kbyte(q0, q1, q2, j) >> 6) << 4);
-  }
-}
-
 // NS: stages in the LDS ring, NS - 1 of them in flight. 3 when the grid takes several workgroups per CU (prefill);
 // deeper rings when few row tiles cover the matrix (short batches), where the stream is latency-bound otherwise.
 // NE: accumulator elements with a live token. Element i holds tokens 8 (i / 4) + i % 4 and 8 (i / 4) + 4 + i % 4 of
@@ -378,7 +362,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_kq(const uint8_t* W, int64_t 
         hd = *reinterpret_cast<const uint4*>(st + S::hdr + gi * 128 + r8 * 16);
       }
       const float d = half_to_float((uint16_t)(hd.x & 0xFFFF)), dmin = half_to_float((uint16_t)(hd.x >> 16));
-      // scale_min_k4 of sub-blocks 4 hf + 0..3, byte u of each word (hd.y, hd.z, hd.w: the 12 packed bytes): the low
+      // scale_min_k4 (the reference's kernels.h:18-26) of sub-blocks 4 hf + 0..3, byte u of each word (hd.y, hd.z, hd.w: the 12 packed bytes): the low
       // half of a super-block takes 6 bits of hd.y / hd.z, the high half nibbles of hd.w and the top bits of those.
       const uint32_t sc4 = hf ? (hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u) : hd.y & 0x3F3F3F3Fu;
       const uint32_t mn4 = hf ? ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u) : hd.z & 0x3F3F3F3Fu;

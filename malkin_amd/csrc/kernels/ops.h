@@ -126,9 +126,9 @@ __host__ __device__ constexpr int kv_perm(int e, int DC) { return DC * (e & 15) 
 // q [n][H*D] (token stride q_stride floats), out [n][H*D] (stride out_stride). Per token t: keys rows
 // 0..n_keys[t]-1 of sequence seq[t], then anc[anc_off[t] .. anc_off[t+1]) when anc_off is non-null. Rows with more
 // keys than one workgroup's LDS holds keep their scores in `scratch` (attention_scratch_bytes of it for full speed;
-// a smaller scratch runs fewer workgroups at a time; one without room for a single row fails). walks: those of the batch,
-// where the host knows seq; else the device finds out where it matters, into *route (a device word of the context; n_seq,
-// the cache's sequences, bounds the batch's).
+// a smaller scratch runs fewer workgroups at a time; one without room for a single row fails). walks: those of the
+// batch, where the host knows seq; else the device finds out where it matters, into *route (a device word of the
+// context; n_seq, the cache's sequences, bounds the batch's).
 struct AttnWalks;             // ctx.h
 constexpr int kRouteMma = 1;  // *route: every token to attention_mma (0: none)
 void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int64_t out_stride, int n, int H, int KV,

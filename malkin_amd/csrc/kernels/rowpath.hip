@@ -271,7 +271,10 @@ __global__ __launch_bounds__(kRowsThreads) void k_gguf45(const uint8_t* __restri
 // DPP. The next pass's row bytes and activations are loaded while this one runs. What bounds it: the vector work of a
 // pass (about 150 instructions per 4 rows x 512 weights, 1408 bytes) and, with few rows, the chain's 32 dependent
 // fmas. Measured against the byte-wise kernel above (8 lanes per row, the dot summed across lanes per sub-block): Q5_K
-// 2560 x 9728 at one token 200 -> 10 us, 19456 x 2560 71 -> 10.8 (3.2 TB/s); at 4 tokens 371 -> 27 and 126 -> 27.
+// 2560 x 9728 at one token 141 -> 9.7 us, 19456 x 2560 71 -> 10.9 (weights in the Infinity Cache; 10.8 and 12.0 between a
+// layer's other matmuls); 2560 x 9728 at 4 tokens 342 -> 26. Q4_K takes it at any count of
+// tokens: 1024 x 3072 at one 44 -> 3.8 us, at 300 218 -> 92, at 512 293 -> 148; 2560 x 9728 at 300 1572 -> 609; 19456 x 2560 at
+// 128 1072 -> 589.
 template <bool kHigh, int NT>
 __global__ __launch_bounds__(kRowsThreads) void k_gguf45_gemv(const uint8_t* __restrict__ W, size_t row_bytes,
                                                               int64_t rows, int64_t cols,

@@ -1,5 +1,5 @@
-"""Grouped attention (head_dim 128, trees) where the heads of a KV group are split over two or three workgroups, also
-unevenly, bit for bit against the oracle's attend_gqa."""
+"""Grouped attention (head_dim 128, trees) where the heads of a KV group are split over two, three or five workgroups,
+also unevenly, bit for bit against the oracle's attend_gqa."""
 import pytest
 
 from test_gpu_kernels import _attention_vs_oracle, _tree

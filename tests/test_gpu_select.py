@@ -1,8 +1,6 @@
 """mk_topk where its forms meet: rows that one workgroup takes alone (up to 8192 logits), rows cut into 64 slices, slices
-of 4, 8, 12 or 16
-logits a thread, slices walked in rounds (more than 4096 logits each), rows whose largest logits fall into one slice
-(the row is then walked whole), and more rows than the context's scratch holds candidates for, against numpy's stable
-order."""
+of 4, 8, 12 or 16 logits a thread, slices walked in rounds (more than 4096 logits each), rows whose largest logits fall
+into a few slices (which are then walked whole), and many rows, against numpy's stable order."""
 import numpy as np
 import pytest
 
