@@ -45,7 +45,8 @@ const char* mk_last_error(void);
 int mk_synchronize(mk_ctx* ctx);
 /* Grows the context's device scratch buffer to at least `bytes` (never shrinks; waits for the stream first). Calls
    that use the scratch (mk_attention on rows longer than one workgroup's LDS, mk_argmax_top2) then run without
-   allocating, also under graph capture. No reference counterpart (the CPU engine's scratch is host memory). */
+   allocating, also under graph capture; a graph captured before the scratch grows keeps the old buffer's address, so
+   reserve first. No reference counterpart (the CPU engine's scratch is host memory). */
 int mk_reserve_scratch(mk_ctx* ctx, size_t bytes);
 /* Scratch mk_attention needs for `pairs` (token, query head) pairs over up to max_keys keys: 0 while a row fits in
    one workgroup's LDS (about 7600 keys at head_dim 128); beyond that, global slots of 2 floats per key per pair
