@@ -1497,27 +1497,29 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
   const int G = H / KV;
   const bool aligned = attn_aligned(a);
   const int GH = grp_heads(n, H, G, D, a, anc_off, max_keys);
-  // Many plain tokens on the matrix cores: always where a row's scores fit LDS. Longer rows, whose scores run twice, where
-  // the batch takes more than two rounds of the CUs otherwise and its walks pay (mma_pays); where only the device knows
-  // the sequences and they matter, it decides: both kernels are launched and one of them leaves at once (4 to 9 us).
-  // Measured at 32 heads over 8 KV heads, the grouped kernel / this, us: 128 tokens of one sequence over 2000 keys
-  // 169 / 92, of 64 sequences 171 / 187, of 128 180 / 366; 128 tokens over 6000 keys, where a group's heads take workgroups
-  // of their own, 1229 / 262, 1233 / 554 and 1238 / 1083; 8 heads over 8 KV heads, 80 tokens of one sequence over 4000 keys
-  // 159 / 177. (Past the grouped kernel's keys the caller's scratch must hold a row all the same: such calls have always
+  // Many plain tokens on the matrix cores: always where a row's scores fit LDS, and longer rows, whose scores run twice,
+  // where the batch's walks pay (mma_pays). Measured at 32 heads over 8 KV heads, the grouped kernel / this, us: 128 tokens
+  // of one sequence over 2000 keys 169 / 92, of 64 sequences 171 / 187, of 128 180 / 366; 128 tokens over 6000 keys, where
+  // a group's heads take workgroups of their own, 1229 / 262, 1233 / 554 and 1238 / 1083; 8 heads over 8 KV heads, 80 tokens
+  // of one sequence over 4000 keys 159 / 177; 64 over 4, 64 tokens over 1880 keys
+  // 420 / 87.
+  // Where only the device knows the sequences and they matter, it decides: both kernels are launched and one of them
+  // leaves at once, which takes 4 to 9 us; batches of two rounds of the CUs or less are not worth that and stay on the
+  // grouped kernel. (Past that one's keys the caller's scratch must hold a row whoever takes it: such calls have always
   // needed it.)
   const int32_t* routed = nullptr;
   if (!anc_off && n >= kRowsMinTokens && attention_mma_ok(G, D, a)) {
     bool mma = attention_mma_whole(max_keys);
-    if (!mma && (int64_t)n * KV > 2 * device_cus() &&
-        (GH > 0 || (scratch && scratch_bytes >= 2 * (size_t)attn_keys_pad(max_keys) * sizeof(float)))) {
+    if (!mma && (GH > 0 || (scratch && scratch_bytes >= 2 * (size_t)attn_keys_pad(max_keys) * sizeof(float)))) {
       const int TQ = kRowsMax / G, nblk = (n + TQ - 1) / TQ, cus = device_cus();
       const int rest = rest_cost(n, KV, G, GH);
       // One sequence a block at best; at worst every token of a block its own (or as many as the cache has).
       const AttnWalks best{nblk, 1}, worst{std::min<int>(n, nblk * std::min(TQ, n_seq)), std::min({TQ, n_seq, n})};
-      mma = mma_pays(walks ? *walks : best, nblk, KV, cus, rest);
-      if (mma && !walks && !mma_pays(worst, nblk, KV, cus, rest)) {
+      mma = mma_pays(walks ? *walks : worst, nblk, KV, cus, rest);
+      if (!mma && !walks && (int64_t)n * KV > 2 * cus && mma_pays(best, nblk, KV, cus, rest)) {
         hipLaunchKernelGGL(k_attention_route, dim3(1), dim3(1024), 0, s, seq, n, TQ, KV, cus, rest, route);
         routed = route;
+        mma = true;
       }
     }
     if (mma) {

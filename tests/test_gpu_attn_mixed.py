@@ -26,6 +26,8 @@ CASES = [  # H, KV, tokens, tokens of sequence 1, tokens of each other one, long
     (24, 8, 73, 73, 1, 1900),    # matrix cores, blocks of 5 tokens
     (40, 8, 71, 71, 1, 1990),    # matrix cores, blocks of 3 tokens
     (16, 1, 520, 520, 1, 1870),  # matrix cores, blocks of one token
+    (48, 8, 64, 20, 1, 1880),    # matrix cores, blocks of 2 tokens
+    (64, 4, 33, 20, 1, 1880),    # matrix cores, blocks of one token
     (32, 8, 70, 33, 1, 2000),    # grouped
     (32, 8, 67, 0, 2, 3000),     # matrix cores, two sequences a block
     (32, 8, 70, 33, 1, 3000),    # grouped, a group's heads in workgroups of their own
