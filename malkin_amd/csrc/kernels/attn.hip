@@ -1501,8 +1501,7 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
   // where the batch's walks pay (mma_pays). Measured at 32 heads over 8 KV heads, the grouped kernel / this, us: 128 tokens
   // of one sequence over 2000 keys 169 / 92, of 64 sequences 171 / 187, of 128 180 / 366; 128 tokens over 6000 keys, where
   // a group's heads take workgroups of their own, 1229 / 262, 1233 / 554 and 1238 / 1083; 8 heads over 8 KV heads, 80 tokens
-  // of one sequence over 4000 keys 159 / 177; 64 over 4, 64 tokens over 1880 keys
-  // 420 / 87.
+  // of one sequence over 4000 keys 159 / 177; 64 over 4, 64 tokens over 1880 keys 420 / 87.
   // Where only the device knows the sequences and they matter, it decides: both kernels are launched and one of them
   // leaves at once, which takes 4 to 9 us; batches of two rounds of the CUs or less are not worth that and stay on the
   // grouped kernel. (Past that one's keys the caller's scratch must hold a row whoever takes it: such calls have always
@@ -1528,7 +1527,7 @@ void attention(hipStream_t s, const float* q, int64_t q_stride, float* out, int6
     }
   }
   if (!anc_off && n >= kRowsMinTokens && G <= 16 && D == 64 && a.k_perm && aligned &&
-             rows_lds_bytes(D, attn_keys_pad(max_keys)) <= 160 * 1024 - 1024) {
+      rows_lds_bytes(D, attn_keys_pad(max_keys)) <= 160 * 1024 - 1024) {
     const int nk_pad = attn_keys_pad(max_keys), TQ = kRowsMax / G;
     allow_lds<k_attention_rows<64>>(kLdsLimit);
     hipLaunchKernelGGL(k_attention_rows<64>, dim3(((n + TQ - 1) / TQ) * KV), dim3(kRowsThreads), rows_lds_bytes(D, nk_pad),
